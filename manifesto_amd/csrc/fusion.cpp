@@ -297,6 +297,8 @@ std::string operand_index(const mfh_operand& op, const char* elem)
     return elem;
 }
 
+bool power_of_two(int64_t v) { return (v & (v - 1)) == 0; }
+
 // ---- compiled-code cache -----------------------------------------------------
 
 struct CodeObject {
@@ -533,7 +535,6 @@ struct mfh_kernel {
     int unroll = 1;  // work items per thread per step
     int block = mfh::kFusedThreads;  // threads per workgroup
     int auto_bpc = 4;  // workgroups per CU unless the launch config sets one
-    bool periods_vectorizable = true;
     std::shared_ptr<mfh::CodeObject> code;
 };
 
@@ -574,10 +575,6 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
             return fail(MFH_ERR_INVALID_ARGUMENT, "codegen hip: input %d period must be positive", k);
         if (op.mode != MFH_OPERAND_SCALAR && op.dtype == kFloat32) vec = 4;
     }
-    bool periods_vectorizable = true;
-    for (int k = 0; k < n_inputs; k++)
-        if (inputs[k].mode == MFH_OPERAND_PERIODIC && inputs[k].period % vec != 0) periods_vectorizable = false;
-
     const bool precise = (flags & MFH_FUSION_PRECISE) != 0;
     // Launch shape: a one-shot grid (one block per `block` x unroll items, so each
     // block streams one chunk and exits and the blocks sweep memory in
@@ -658,30 +655,58 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
         if (inputs[k].mode == MFH_OPERAND_SCALAR)
             src += "    const float s" + std::to_string(k) + " = mfh_ld1_" + io_suffix(inputs[k].dtype) + "(p" +
                    std::to_string(k) + ", 0);\n";
-    // vector loop: loads of all items first, then compute and store
+    // Vector loop: loads of all items first, then compute and store, at any
+    // element alignment of the buffers (mfh_u32x4_any).
+    //
+    // A periodic row of P elements is read at the item's index in it.  Where P
+    // is not a power of two the index takes mfh_row_index (a scalar remainder
+    // per wave and a 32-bit one per lane).  Where P is not a multiple of the
+    // item either, an item that runs over the row's end loads the row's last
+    // whole item instead and is filled element by element afterwards, a
+    // branch that one item in P / vec takes.  The element loop, one 2-byte
+    // access per lane, took 77 us for bias + gelu + residual over bf16
+    // [8190, 2730] on MI355X, this loop 24; silu(gate) * up over bf16 buffers
+    // one element off 16 bytes 58 us against 19.5 (16.5 aligned: a wave's
+    // span then touches one more 128-byte line).
     src += "    for (mfh_i64 v = tid; v < nvec; v += stride * " + U + ") {\n";
+    auto row_ends = [&](int k) { return inputs[k].mode == MFH_OPERAND_PERIODIC && inputs[k].period % vec != 0; };
     for (int k = 0; k < n_inputs; k++) {
         if (inputs[k].mode == MFH_OPERAND_SCALAR) continue;
-        if (packed16[k]) src += "        mfh_u32 w" + std::to_string(k) + "[" + U + "][" + std::to_string(vec / 2) + "];\n";
-        else src += "        float a" + std::to_string(k) + "[" + U + "][" + V + "];\n";
+        const std::string ks = std::to_string(k);
+        if (packed16[k]) src += "        mfh_u32 w" + ks + "[" + U + "][" + std::to_string(vec / 2) + "];\n";
+        else src += "        float a" + ks + "[" + U + "][" + V + "];\n";
+        if (row_ends(k)) src += "        mfh_u64 row" + ks + "[" + U + "];\n";
     }
     src += "#pragma unroll\n        for (int u = 0; u < " + U + "; u++) {\n";
     src += "            const mfh_i64 it = v + u * stride;\n            if (it < nvec) {\n";
     src += "                const mfh_i64 e0 = it * " + V + ";\n";
+    std::string fills;  // of items that run over the end of a periodic row
     for (int k = 0; k < n_inputs; k++) {
         if (inputs[k].mode == MFH_OPERAND_SCALAR) continue;
-        std::string ks = std::to_string(k);
+        const std::string ks = std::to_string(k), sfx = io_suffix(inputs[k].dtype);
         const std::string nt = stream_loads && inputs[k].mode == MFH_OPERAND_FULL ? "<1>" : "";
-        if (packed16[k])
-            src += "                mfh_ldw" + V + "_f16" + nt + "(p" + ks + ", " + operand_index(inputs[k], "e0") +
-                   ", w" + ks + "[u]);\n";
-        else
-            src += "                mfh_ld" + V + "_" + io_suffix(inputs[k].dtype) + nt + "(p" + ks + ", " +
-                   operand_index(inputs[k], "e0") + ", a" + ks + "[u]);\n";
+        const std::string to = packed16[k] ? "w" + ks + "[u]" : "a" + ks + "[u]";
+        const int64_t period = inputs[k].period;
+        std::string index = operand_index(inputs[k], "e0");
+        if (inputs[k].mode == MFH_OPERAND_PERIODIC && !power_of_two(period))
+            index = "mfh_row_index<" + std::to_string(period) + "ull>(e0)";
+        if (row_ends(k)) {
+            const std::string row = "row" + ks + "[u]";
+            src += "                " + row + " = " + index + ";\n";
+            const std::string last = std::to_string(period - vec) + "ull";
+            fills += "            if (" + (period >= vec ? row + " > " + last : std::string("true")) + ") mfh_fill" + V + "_" +
+                     (packed16[k] ? "w" : "") + sfx + "<" + std::to_string(period) + "ull>(p" + ks + ", " + row + ", " +
+                     to + ");\n";
+            if (period < vec) continue;  // no whole item in the row: filled only
+            index = "(" + row + " < " + last + " ? " + row + " : " + last + ")";
+        }
+        src += std::string("                mfh_ld") + (packed16[k] ? "w" : "") + V + "_" + sfx + nt + "(p" + ks + ", " +
+               index + ", " + to + ");\n";
     }
     src += "            }\n        }\n";
     src += "#pragma unroll\n        for (int u = 0; u < " + U + "; u++) {\n";
     src += "            const mfh_i64 it = v + u * stride;\n            if (it >= nvec) break;\n";
+    src += fills;
     std::string operands;
     for (int k = 0; k < n_inputs; k++) {
         std::string ks = std::to_string(k);
@@ -735,7 +760,6 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     kernel->unroll = unroll;
     kernel->block = block;
     kernel->auto_bpc = auto_bpc;
-    kernel->periods_vectorizable = periods_vectorizable;
     MFH_TRY(compile_source(kernel->source, kernel_name, &kernel->code));
     *out = kernel.release();
     return MFH_OK;
@@ -764,16 +788,15 @@ int prepare_hip(const mfh_kernel* kernel, const void* const* inputs, int n_input
     MFH_TRY(bind_device(&dev));
     if (count == 0) return MFH_OK;
     if (!out) return fail(MFH_ERR_INVALID_ARGUMENT, "codegen hip: output buffer is NULL");
-    // The vector path needs every streamed buffer aligned to one item's bytes.
-    auto item_aligned = [&](const void* p, int dtype) {
-        uintptr_t bytes = (uintptr_t)kernel->vec * (dtype == kFloat32 ? 4 : 2);
-        return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0;
+    // The vector path reads and writes whole items at any element alignment.
+    auto element_aligned = [](const void* p, int dtype) {
+        return (reinterpret_cast<uintptr_t>(p) & (dtype == kFloat32 ? 3u : 1u)) == 0;
     };
-    bool vec_ok = kernel->periods_vectorizable && item_aligned(out, kernel->out_dtype);
+    bool vec_ok = element_aligned(out, kernel->out_dtype);
     for (int k = 0; k < n_inputs; k++) {
         if (!inputs[k])
             return fail(MFH_ERR_INVALID_ARGUMENT, "codegen hip: input %d is NULL", k);
-        if (kernel->inputs[k].mode != MFH_OPERAND_SCALAR && !item_aligned(inputs[k], kernel->inputs[k].dtype))
+        if (kernel->inputs[k].mode != MFH_OPERAND_SCALAR && !element_aligned(inputs[k], kernel->inputs[k].dtype))
             vec_ok = false;
     }
     MFH_TRY(load_function(*kernel->code, dev->ordinal, may_load, &launch->fn));
