@@ -52,8 +52,6 @@ struct Device {
 // MFH_ERR_NOT_INITIALIZED when mfh_init has not run.
 int bind_device(const Device** out);
 
-inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
-
 // Streaming kernels with their own grid-size setting.
 enum class Kern { kFp8, kInt4, kAxpy, kAxpy16, kConvert, kFused, kCount };
 

@@ -5,9 +5,11 @@
 // neighbours, so each store instruction of a wave writes 1 KiB contiguously
 // and each load instruction reads a contiguous span.  Threads take U items
 // per step (loads first, then converts and stores): FP8 in one-shot chunks
-// per workgroup, the others in grid-stride loops.  A scalar loop finishes the
-// elements after the last whole item, and does all of them when a pointer is
-// not aligned for the vector path.
+// per workgroup, the others in grid-stride loops.  An element loop finishes
+// the elements after the last whole item.  Buffers may stand at any byte
+// address (launch.hpp).  One element off 16 bytes, 2^24 elements on MI355X:
+// FP8 -> bf16 10.3 us (26.5 by element loops with 1- and 2-byte accesses),
+// f32 -> bf16 17.8 (35.6), bf16 -> f32 16.0 (37.9), int8 -> f32 13.0 (22.8).
 //
 // FP8: the output for a code depends only on (code, format, scale), so each
 // workgroup first builds the 256-entry table in LDS with the exact rules of
@@ -76,13 +78,13 @@ MFH_DEV mfh_u32 fp8_bits_hw(mfh_u32 code, bool e5m2)
 template <int OUT, int U, int BS>
 __global__ __launch_bounds__(BS) void k_dequant_fp8(const mfh_u8* __restrict__ in,
                                                         void* __restrict__ out, mfh_i64 n,
-                                                        float scale, int fmt, int vec_ok)
+                                                        float scale, int fmt)
 {
     __shared__ mfh_u32 lut[256];
     constexpr int kCodes = OUT == kFloat32 ? 4 : 8;
     constexpr mfh_i64 kChunk = (mfh_i64)BS * U;
     const mfh_u32 t = threadIdx.x;
-    const mfh_i64 nitems = vec_ok ? n / kCodes : 0;
+    const mfh_i64 nitems = n / kCodes;
     const mfh_i64 nchunks = (nitems + kChunk - 1) / kChunk;
     u32x2 w[U];
     auto load = [&](mfh_i64 c) {
@@ -90,8 +92,8 @@ __global__ __launch_bounds__(BS) void k_dequant_fp8(const mfh_u8* __restrict__ i
         for (int u = 0; u < U; u++) {
             const mfh_i64 i = c * kChunk + u * BS + t;
             if (i < nitems) {
-                if constexpr (kCodes == 8) w[u] = load_nt(&reinterpret_cast<const u32x2*>(in)[i]);
-                else w[u] = u32x2{reinterpret_cast<const mfh_u32*>(in)[i], 0u};
+                if constexpr (kCodes == 8) w[u] = load8<true>(in + i * 8);
+                else w[u] = u32x2{load4(in + i * 4), 0u};
             }
         }
     };
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(BS) void k_dequant_fp8(const mfh_u8* __restrict__ i
     for (; c < nchunks; c += gridDim.x) {
         if (c != (mfh_i64)blockIdx.x) load(c);
         const mfh_i64 first = c * kChunk;
-        const StreamOut dst(reinterpret_cast<u32x4*>(out) + first, nitems - first);
+        const StreamOut dst(static_cast<char*>(out) + first * 16, nitems - first);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int j = u * BS + (int)t;
@@ -206,8 +208,8 @@ __global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ 
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const mfh_u32 j = (mfh_u32)min(u * BS + t, last);
-            if constexpr (kElems == 8) w[u] = *reinterpret_cast<const mfh_u32*>(items + j * kItemBytes);
-            else w[u] = *reinterpret_cast<const mfh_u16*>(items + j * kItemBytes);
+            if constexpr (kElems == 8) w[u] = load4(items + j * kItemBytes);
+            else w[u] = load2(items + j * kItemBytes);
             sb[u] = scale_bits<SDT>(group0 + ((gr + j * kElems) >> gs) * kScaleBytes, 0);
         }
         __builtin_amdgcn_sched_barrier(0);  // every load of the chunk ahead of the first wait
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ 
 #pragma unroll
         for (int u = 0; u < U; u++) s[u] = scale_value<SDT>(sb[u]);
         // The buffer descriptor ends at the last item: stores past it are dropped.
-        const StreamOut dst(reinterpret_cast<u32x4*>(out) + first, nitems - first);
+        const StreamOut dst(static_cast<char*>(out) + first * 16, nitems - first);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int j = u * BS + t;
@@ -274,61 +276,6 @@ MFH_DEV float decode_at(const void* in, mfh_i64 i)
     else return (float)static_cast<const mfh_u8*>(in)[i];
 }
 
-template <int IN, int OUT>
-__global__ __launch_bounds__(kBlock) void k_convert(const void* __restrict__ in, void* __restrict__ out,
-                                                    mfh_i64 n)
-{
-    const mfh_i64 stride = (mfh_i64)gridDim.x * kBlock;
-    for (mfh_i64 i = (mfh_i64)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
-        store_one<OUT>(out, i, encode_one<OUT>(decode_at<IN>(in, i)));
-}
-
-template <int IN>
-MFH_DEV float dec16(mfh_u32 h)
-{
-    return IN == kBFloat16 ? mfh_bf16_to_f32(h) : mfh_f16_to_f32(h);
-}
-
-// 16-bit storage -> any output, one 16-byte store per item: 8 elements for a
-// 16-bit output, 4 for f32.  (The cast that sits between a bf16/f16 tensor and
-// an f32 fusion in the reference.)
-template <int IN, int OUT, int BS, int U>
-__global__ __launch_bounds__(BS) void k_convert16_vec(const void* __restrict__ in, void* __restrict__ out,
-                                                          mfh_i64 nitems)
-{
-    const mfh_i64 chunk = (mfh_i64)BS * U;  // items of a workgroup, thread t holding t, t + BS, ...
-    u32x4* dst = reinterpret_cast<u32x4*>(out);
-    for (mfh_i64 base = (mfh_i64)blockIdx.x * chunk; base < nitems; base += (mfh_i64)gridDim.x * chunk) {
-        if constexpr (OUT == kFloat32) {
-            u32x2 w[U];
-#pragma unroll
-            for (int u = 0; u < U; u++)  // past-the-end items load the last one again
-                w[u] = reinterpret_cast<const u32x2*>(in)[min(base + u * BS + (mfh_i64)threadIdx.x, nitems - 1)];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const mfh_i64 v = base + u * BS + (mfh_i64)threadIdx.x;
-                if (v < nitems)
-                    store_nt(&dst[v], u32x4{mfh_bits(dec16<IN>(w[u][0] & 0xffffu)), mfh_bits(dec16<IN>(w[u][0] >> 16)),
-                                            mfh_bits(dec16<IN>(w[u][1] & 0xffffu)), mfh_bits(dec16<IN>(w[u][1] >> 16))});
-            }
-        } else {
-            u32x4 w[U];
-#pragma unroll
-            for (int u = 0; u < U; u++)
-                w[u] = load_nt(reinterpret_cast<const u32x4*>(in) + min(base + u * BS + (mfh_i64)threadIdx.x, nitems - 1));
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                const mfh_i64 v = base + u * BS + (mfh_i64)threadIdx.x;
-                u32x4 o;
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    o[k] = encode_pair<OUT>(dec16<IN>(w[u][k] & 0xffffu), dec16<IN>(w[u][k] >> 16));
-                if (v < nitems) store_nt(&dst[v], o);
-            }
-        }
-    }
-}
-
 // Byte size of an unpacked numeric dtype, at compile time.
 template <int DT>
 constexpr int size_of()
@@ -383,7 +330,7 @@ __global__ __launch_bounds__(BS) void k_convert_vec(const void* __restrict__ in,
     constexpr int W = B / 4;                        // source dwords per item
     const mfh_i64 nitems = n / E;
     const mfh_i64 chunk = (mfh_i64)BS * U;          // items of a workgroup, thread t holding t, t + BS, ...
-    u32x4* dst = reinterpret_cast<u32x4*>(out);
+    u32x4_any* dst = static_cast<u32x4_any*>(out);
     for (mfh_i64 base = (mfh_i64)blockIdx.x * chunk; base < nitems; base += (mfh_i64)gridDim.x * chunk) {
         mfh_u32 w[U][W];
 #pragma unroll
@@ -395,14 +342,14 @@ __global__ __launch_bounds__(BS) void k_convert_vec(const void* __restrict__ in,
             if constexpr (B >= 16) {
 #pragma unroll
                 for (int q = 0; q < B / 16; q++) {
-                    const u32x4 x = load_nt(reinterpret_cast<const u32x4*>(src) + q);
+                    const u32x4 x = load16<true>(src + 16 * q);
                     w[u][4 * q] = x[0], w[u][4 * q + 1] = x[1], w[u][4 * q + 2] = x[2], w[u][4 * q + 3] = x[3];
                 }
             } else if constexpr (B == 8) {
-                const u32x2 x = *reinterpret_cast<const u32x2*>(src);
+                const u32x2 x = load8<false>(src);
                 w[u][0] = x[0], w[u][1] = x[1];
             } else {
-                w[u][0] = *reinterpret_cast<const mfh_u32*>(src);
+                w[u][0] = load4(src);
             }
         }
 #pragma unroll
@@ -417,7 +364,7 @@ __global__ __launch_bounds__(BS) void k_convert_vec(const void* __restrict__ in,
                     o[k] = encode_pair<OUT>(decode_reg<IN>(w[u], 2 * k), decode_reg<IN>(w[u], 2 * k + 1));
             }
             const mfh_i64 v = base + u * BS + (mfh_i64)threadIdx.x;
-            if (v < nitems) store_nt(&dst[v], o);
+            if (v < nitems) store16(&dst[v], o);
         }
     }
     const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
@@ -425,28 +372,15 @@ __global__ __launch_bounds__(BS) void k_convert_vec(const void* __restrict__ in,
         store_one<OUT>(out, i, encode_one<OUT>(decode_at<IN>(in, i)));
 }
 
-// f32 -> 16-bit storage, 4 elements per item (16-byte load, 8-byte store).
-template <int OUT, int BS>
-__global__ __launch_bounds__(BS) void k_narrow_f32_vec(const u32x4* __restrict__ in,
-                                                           u32x2* __restrict__ out, mfh_i64 nitems)
-{
-    const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
-    for (mfh_i64 v = (mfh_i64)blockIdx.x * BS + threadIdx.x; v < nitems; v += stride) {
-        u32x4 a = load_nt(in + v);
-        store_nt(&out[v], u32x2{encode_pair<OUT>(mfh_f32(a[0]), mfh_f32(a[1])),
-                                encode_pair<OUT>(mfh_f32(a[2]), mfh_f32(a[3]))});
-    }
-}
-
-// Sources wider than the output (8-byte -> f32 / bf16 / f16, 4-byte integers
-// -> bf16 / f16): one 16-byte source piece per lane per step, its 16 / S
+// Sources wider than the output (8-byte -> f32 / bf16 / f16, 4-byte ->
+// bf16 / f16): one 16-byte source piece per lane per step, its 16 / S
 // elements stored together (a 4- or 8-byte store), so that every load
 // instruction reads 1 KiB contiguously.  The generic item layout, which
 // loads two or four adjacent 16-byte pieces per 16-byte store, ran f64 ->
 // f32 at 6.19 TB/s against 6.9 this way.  The last n % (16 / S) elements are
 // the first workgroup's.
 template <int IN, int OUT, int BS>
-__global__ __launch_bounds__(BS) void k_narrow_vec(const u32x4* __restrict__ in, void* __restrict__ out, mfh_i64 n)
+__global__ __launch_bounds__(BS) void k_narrow_vec(const void* __restrict__ in, void* __restrict__ out, mfh_i64 n)
 {
     constexpr int S = size_of<IN>();
     constexpr int E = 16 / S;  // elements per piece: 2 or 4
@@ -454,23 +388,21 @@ __global__ __launch_bounds__(BS) void k_narrow_vec(const u32x4* __restrict__ in,
     const mfh_i64 npieces = n / E;
     const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
     for (mfh_i64 v = (mfh_i64)blockIdx.x * BS + threadIdx.x; v < npieces; v += stride) {
-        const u32x4 a = load_nt(in + v);
+        const u32x4 a = load16<true>(static_cast<const u32x4_any*>(in) + v);
         const mfh_u32 w[4] = {a[0], a[1], a[2], a[3]};
         if constexpr (OUT == kFloat32) {
             static_assert(E == 2, "f32 output from 8-byte sources");
-            store_nt(static_cast<u32x2*>(out) + v, u32x2{mfh_bits(decode_reg<IN>(w, 0)), mfh_bits(decode_reg<IN>(w, 1))});
+            store8(static_cast<u32x2_any*>(out) + v, u32x2{mfh_bits(decode_reg<IN>(w, 0)), mfh_bits(decode_reg<IN>(w, 1))});
         } else if constexpr (E == 2) {
-            store_nt(static_cast<mfh_u32*>(out) + v, encode_pair<OUT>(decode_reg<IN>(w, 0), decode_reg<IN>(w, 1)));
+            store4(static_cast<u32_any*>(out) + v, encode_pair<OUT>(decode_reg<IN>(w, 0), decode_reg<IN>(w, 1)));
         } else {
-            store_nt(static_cast<u32x2*>(out) + v, u32x2{encode_pair<OUT>(decode_reg<IN>(w, 0), decode_reg<IN>(w, 1)),
+            store8(static_cast<u32x2_any*>(out) + v, u32x2{encode_pair<OUT>(decode_reg<IN>(w, 0), decode_reg<IN>(w, 1)),
                                                          encode_pair<OUT>(decode_reg<IN>(w, 2), decode_reg<IN>(w, 3))});
         }
     }
     const mfh_i64 i = npieces * E + threadIdx.x;
     if (blockIdx.x == 0 && threadIdx.x < E && i < n) store_one<OUT>(out, i, encode_one<OUT>(decode_at<IN>(in, i)));
 }
-
-bool aligned(const void* p, unsigned bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; }
 
 // ---------------------------------------------------------------------------
 // Any numeric dtype -> one byte per element: FP8 (BytesToFloat8E4M3 /
@@ -564,25 +496,31 @@ MFH_DEV mfh_u32 word_at(const void* in, mfh_i64 e0)
     }
 }
 
-// FP8 and Int4 sources, and any source whose buffers are not aligned for
-// k_encode_byte_wave: item = 16 elements decoded one by one -> one 16-byte
-// store of codes when the output is 16-byte aligned, else the element loop.
+// FP8 and Int4 sources: item = 16 elements decoded one by one -> one 16-byte
+// store of codes.
 template <int IN, int ENC>
 __global__ __launch_bounds__(kBlock) void k_encode_byte(const void* __restrict__ in, mfh_u8* __restrict__ out,
-                                                        mfh_i64 n, int vec_ok)
+                                                        mfh_i64 n)
 {
     const mfh_i64 stride = (mfh_i64)gridDim.x * kBlock;
-    const mfh_i64 nitems = vec_ok ? n / 16 : 0;
-    u32x4* dst = reinterpret_cast<u32x4*>(out);
+    const mfh_i64 nitems = n / 16;
+    u32x4_any* dst = reinterpret_cast<u32x4_any*>(out);
     for (mfh_i64 v = (mfh_i64)blockIdx.x * kBlock + threadIdx.x; v < nitems; v += stride) {
         u32x4 o;
 #pragma unroll
         for (int q = 0; q < 4; q++) o[q] = word_at<IN, ENC>(in, v * 16 + 4 * q);
-        store_nt(&dst[v], o);
+        store16(&dst[v], o);
     }
     for (mfh_i64 i = nitems * 16 + (mfh_i64)blockIdx.x * kBlock + threadIdx.x; i < n; i += stride)
         out[i] = (mfh_u8)byte_at<IN, ENC>(in, i);
 }
+
+// Whether the encoders stream their source (non-temporal loads).  Where it
+// stands off 16 bytes every wave shares the lines at its span's ends with its
+// neighbours, and plain loads, which leave them in the cache, run bf16 ->
+// e4m3 of 2^24 elements read a moment before in 9.7 against 11.1 us (11.6
+// against 11.4 from HBM).
+bool streamed_source(const void* in) { return (reinterpret_cast<uintptr_t>(in) & 15u) == 0; }
 
 // Unpacked numeric dtype -> one byte per element with every load instruction
 // of a wave reading 1 KiB contiguously: a wave takes chunks of 4 KiB of
@@ -594,7 +532,7 @@ __global__ __launch_bounds__(kBlock) void k_encode_byte(const void* __restrict__
 // taking 16 consecutive elements (64 bytes of f32) spreads each load
 // instruction over 4 KiB: f32 -> e4m3 ran at 4.4 TB/s that way.  Elements
 // past the last whole chunk run the element loop.
-template <int IN, int ENC, int BS>
+template <int IN, int ENC, int BS, bool NT>
 __global__ __launch_bounds__(BS) void k_encode_byte_wave(const void* __restrict__ in, mfh_u8* __restrict__ out,
                                                              mfh_i64 n)
 {
@@ -609,18 +547,18 @@ __global__ __launch_bounds__(BS) void k_encode_byte_wave(const void* __restrict_
         u32x4 x[kPieces];
 #pragma unroll
         for (int q = 0; q < kPieces; q++)
-            x[q] = load_nt(reinterpret_cast<const u32x4*>(in) + c * (64 * kPieces) + q * 64 + lane);
+            x[q] = load16<NT>(static_cast<const u32x4_any*>(in) + c * (64 * kPieces) + q * 64 + lane);
 #pragma unroll
         for (int q = 0; q < kPieces; q++) {
             const mfh_u32 w[4] = {x[q][0], x[q][1], x[q][2], x[q][3]};
             mfh_u32 code[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
             for (int j = 0; j < (P + 3) / 4; j++) code[j] = word_reg<IN, ENC, P>(w, j);
-            const mfh_i64 e0 = c * kChunk + (mfh_i64)(q * 64 + lane) * P;
-            if constexpr (P == 16) store_nt(reinterpret_cast<u32x4*>(out + e0), u32x4{code[0], code[1], code[2], code[3]});
-            else if constexpr (P == 8) store_nt(reinterpret_cast<u32x2*>(out + e0), u32x2{code[0], code[1]});
-            else if constexpr (P == 4) store_nt(reinterpret_cast<mfh_u32*>(out + e0), code[0]);
-            else store_nt(reinterpret_cast<mfh_u16*>(out + e0), (mfh_u16)code[0]);
+            mfh_u8* o = out + c * kChunk + (mfh_i64)(q * 64 + lane) * P;
+            if constexpr (P == 16) store16(o, u32x4{code[0], code[1], code[2], code[3]});
+            else if constexpr (P == 8) store8(o, u32x2{code[0], code[1]});
+            else if constexpr (P == 4) store4(o, code[0]);
+            else store2(o, code[0]);
         }
     }
     const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
@@ -649,7 +587,10 @@ int launch_encode_byte_wave(const Device* dev, mfh_u8* out, const void* in, int 
     const unsigned grid = grid_for(std::max<int64_t>(n / chunk_elems, 1) * 64, dev, Kern::kConvert, 1, BS);
     switch (in_dt) {
 #define MFH_ENCODE_WAVE_CASE(DT) \
-    case DT: k_encode_byte_wave<DT, ENC, BS><<<grid, BS, 0, stream>>>(in, out, n); break;
+    case DT: \
+        if (streamed_source(in)) k_encode_byte_wave<DT, ENC, BS, true><<<grid, BS, 0, stream>>>(in, out, n); \
+        else k_encode_byte_wave<DT, ENC, BS, false><<<grid, BS, 0, stream>>>(in, out, n); \
+        break;
         MFH_ENCODE_WAVE_CASE(kFloat64)
         MFH_ENCODE_WAVE_CASE(kFloat32)
         MFH_ENCODE_WAVE_CASE(kFloat16)
@@ -672,35 +613,19 @@ int launch_encode_byte_wave(const Device* dev, mfh_u8* out, const void* in, int 
 template <int ENC>
 int launch_encode_byte(const Device* dev, mfh_u8* out, const void* in, int in_dt, int64_t n, hipStream_t stream)
 {
-    // unpacked numeric sources: whole 4 KiB source chunks per wave when the
-    // source is 16-byte aligned and the output aligned for the kernel's
-    // stores (16 / size bytes)
+    // unpacked numeric sources: whole 4 KiB source chunks per wave
     const int size = in_dt == kF8E4M3 || in_dt == kF8E5M2 || in_dt == kInt4 ? 0 : dtype_size(in_dt);
-    if (size > 0 && aligned16(in) && (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(16 / size - 1)) == 0)
+    if (size > 0)
         return with_block(cast_threads(in_dt, 1), [&](auto block) {
             return launch_encode_byte_wave<ENC, decltype(block)::value>(dev, out, in, in_dt, n, size, stream);
         });
-    const int vec_ok = aligned16(out) && n >= 16;
-    const int64_t items = vec_ok ? n / 16 : n;
-    const unsigned grid = grid_for(items, dev, Kern::kConvert);
+    const unsigned grid = grid_for(std::max<int64_t>(n / 16, 1), dev, Kern::kConvert);
     switch (in_dt) {
 #define MFH_ENCODE_CASE(DT) \
-    case DT: k_encode_byte<DT, ENC><<<grid, kBlock, 0, stream>>>(in, out, n, vec_ok); break;
-        MFH_ENCODE_CASE(kFloat64)
-        MFH_ENCODE_CASE(kFloat32)
-        MFH_ENCODE_CASE(kFloat16)
-        MFH_ENCODE_CASE(kBFloat16)
+    case DT: k_encode_byte<DT, ENC><<<grid, kBlock, 0, stream>>>(in, out, n); break;
         MFH_ENCODE_CASE(kF8E4M3)
         MFH_ENCODE_CASE(kF8E5M2)
-        MFH_ENCODE_CASE(kInt64)
-        MFH_ENCODE_CASE(kInt32)
-        MFH_ENCODE_CASE(kInt16)
-        MFH_ENCODE_CASE(kInt8)
         MFH_ENCODE_CASE(kInt4)
-        MFH_ENCODE_CASE(kUint64)
-        MFH_ENCODE_CASE(kUint32)
-        MFH_ENCODE_CASE(kUint16)
-        MFH_ENCODE_CASE(kUint8)
 #undef MFH_ENCODE_CASE
     default:
         return fail(MFH_ERR_DTYPE_UNSUPPORTED, "mfh_convert: input dtype %s is not supported", dtype_name(in_dt));
@@ -755,15 +680,15 @@ MFH_DEV mfh_u32 nibble_reg(const mfh_u32* w, int k)
     return (mfh_u32)v & 0xfu;
 }
 
-// Item = 32 elements -> one 16-byte store of nibbles (16-byte aligned
-// output), then the byte loop for the rest.
+// FP8 and Int4 sources: item = 32 elements -> one 16-byte store of nibbles,
+// then the byte loop for the rest.
 template <int IN>
 __global__ __launch_bounds__(kBlock) void k_encode_int4(const void* __restrict__ in, mfh_u8* __restrict__ out,
-                                                        mfh_i64 n, int vec_ok)
+                                                        mfh_i64 n)
 {
     const mfh_i64 stride = (mfh_i64)gridDim.x * kBlock;
-    const mfh_i64 nitems = vec_ok ? n / 32 : 0;
-    u32x4* dst = reinterpret_cast<u32x4*>(out);
+    const mfh_i64 nitems = n / 32;
+    u32x4_any* dst = reinterpret_cast<u32x4_any*>(out);
     for (mfh_i64 v = (mfh_i64)blockIdx.x * kBlock + threadIdx.x; v < nitems; v += stride) {
         u32x4 o;
 #pragma unroll
@@ -773,7 +698,7 @@ __global__ __launch_bounds__(kBlock) void k_encode_int4(const void* __restrict__
             for (int k = 0; k < 8; k++) word |= nibble_at<IN>(in, v * 32 + 8 * q + k) << (4 * k);
             o[q] = word;
         }
-        store_nt(&dst[v], o);
+        store16(&dst[v], o);
     }
     const mfh_i64 nbytes = (n + 1) / 2;
     for (mfh_i64 b = nitems * 16 + (mfh_i64)blockIdx.x * kBlock + threadIdx.x; b < nbytes; b += stride) {
@@ -788,7 +713,7 @@ __global__ __launch_bounds__(kBlock) void k_encode_int4(const void* __restrict__
 // every load instruction reads 1 KiB contiguously; the 16 / size elements of
 // a piece leave as 8 / size bytes of nibbles next to the neighbours' ones.
 // Elements past the last whole chunk run the byte loop.
-template <int IN, int BS>
+template <int IN, int BS, bool NT>
 __global__ __launch_bounds__(BS) void k_encode_int4_wave(const void* __restrict__ in, mfh_u8* __restrict__ out,
                                                              mfh_i64 n)
 {
@@ -802,7 +727,8 @@ __global__ __launch_bounds__(BS) void k_encode_int4_wave(const void* __restrict_
     for (mfh_i64 c = (mfh_i64)blockIdx.x * (BS / 64) + (threadIdx.x >> 6); c < nchunks; c += waves) {
         u32x4 x[kPieces];
 #pragma unroll
-        for (int q = 0; q < kPieces; q++) x[q] = load_nt(reinterpret_cast<const u32x4*>(in) + c * (64 * kPieces) + q * 64 + lane);
+        for (int q = 0; q < kPieces; q++)
+            x[q] = load16<NT>(static_cast<const u32x4_any*>(in) + c * (64 * kPieces) + q * 64 + lane);
 #pragma unroll
         for (int q = 0; q < kPieces; q++) {
             const mfh_u32 w[4] = {x[q][0], x[q][1], x[q][2], x[q][3]};
@@ -810,9 +736,9 @@ __global__ __launch_bounds__(BS) void k_encode_int4_wave(const void* __restrict_
 #pragma unroll
             for (int k = 0; k < P; k++) code[k >> 3] |= nibble_reg<IN>(w, k) << (4 * (k & 7));
             mfh_u8* o = out + (c * kChunk + (mfh_i64)(q * 64 + lane) * P) / 2;
-            if constexpr (P == 16) store_nt(reinterpret_cast<u32x2*>(o), u32x2{code[0], code[1]});
-            else if constexpr (P == 8) store_nt(reinterpret_cast<mfh_u32*>(o), code[0]);
-            else if constexpr (P == 4) store_nt(reinterpret_cast<mfh_u16*>(o), (mfh_u16)code[0]);
+            if constexpr (P == 16) store8(o, u32x2{code[0], code[1]});
+            else if constexpr (P == 8) store4(o, code[0]);
+            else if constexpr (P == 4) store2(o, code[0]);
             else *o = (mfh_u8)code[0];
         }
     }
@@ -833,7 +759,10 @@ int launch_encode_int4_wave(const Device* dev, mfh_u8* out, const void* in, int 
     const unsigned grid = grid_for(std::max<int64_t>(n / chunk_elems, 1) * 64, dev, Kern::kConvert, 1, BS);
     switch (in_dt) {
 #define MFH_ENCODE_I4_WAVE_CASE(DT) \
-    case DT: k_encode_int4_wave<DT, BS><<<grid, BS, 0, stream>>>(in, out, n); break;
+    case DT: \
+        if (streamed_source(in)) k_encode_int4_wave<DT, BS, true><<<grid, BS, 0, stream>>>(in, out, n); \
+        else k_encode_int4_wave<DT, BS, false><<<grid, BS, 0, stream>>>(in, out, n); \
+        break;
         MFH_ENCODE_I4_WAVE_CASE(kFloat64)
         MFH_ENCODE_I4_WAVE_CASE(kFloat32)
         MFH_ENCODE_I4_WAVE_CASE(kFloat16)
@@ -855,34 +784,19 @@ int launch_encode_int4_wave(const Device* dev, mfh_u8* out, const void* in, int 
 
 int launch_encode_int4(const Device* dev, mfh_u8* out, const void* in, int in_dt, int64_t n, hipStream_t stream)
 {
-    // unpacked numeric sources aligned to 16 bytes, the output aligned to one
-    // piece's bytes of nibbles (8 / size), take the wave layout
+    // unpacked numeric sources take the wave layout
     const int size = in_dt == kF8E4M3 || in_dt == kF8E5M2 || in_dt == kInt4 ? 0 : dtype_size(in_dt);
-    if (size > 0 && aligned16(in) && (reinterpret_cast<uintptr_t>(out) & (uintptr_t)(std::max(1, 8 / size) - 1)) == 0)
+    if (size > 0)
         return with_block(cast_threads(in_dt, 1), [&](auto block) {
             return launch_encode_int4_wave<decltype(block)::value>(dev, out, in, in_dt, n, size, stream);
         });
-    const int vec_ok = aligned16(out) && n >= 32;
-    const int64_t items = vec_ok ? n / 32 : (n + 1) / 2;
-    const unsigned grid = grid_for(items, dev, Kern::kConvert);
+    const unsigned grid = grid_for(std::max<int64_t>(n / 32, 1), dev, Kern::kConvert);
     switch (in_dt) {
 #define MFH_ENCODE_I4_CASE(DT) \
-    case DT: k_encode_int4<DT><<<grid, kBlock, 0, stream>>>(in, out, n, vec_ok); break;
-        MFH_ENCODE_I4_CASE(kFloat64)
-        MFH_ENCODE_I4_CASE(kFloat32)
-        MFH_ENCODE_I4_CASE(kFloat16)
-        MFH_ENCODE_I4_CASE(kBFloat16)
+    case DT: k_encode_int4<DT><<<grid, kBlock, 0, stream>>>(in, out, n); break;
         MFH_ENCODE_I4_CASE(kF8E4M3)
         MFH_ENCODE_I4_CASE(kF8E5M2)
-        MFH_ENCODE_I4_CASE(kInt64)
-        MFH_ENCODE_I4_CASE(kInt32)
-        MFH_ENCODE_I4_CASE(kInt16)
-        MFH_ENCODE_I4_CASE(kInt8)
         MFH_ENCODE_I4_CASE(kInt4)
-        MFH_ENCODE_I4_CASE(kUint64)
-        MFH_ENCODE_I4_CASE(kUint32)
-        MFH_ENCODE_I4_CASE(kUint16)
-        MFH_ENCODE_I4_CASE(kUint8)
 #undef MFH_ENCODE_I4_CASE
     default:
         return fail(MFH_ERR_DTYPE_UNSUPPORTED, "mfh_convert: input dtype %s is not supported", dtype_name(in_dt));
@@ -930,7 +844,7 @@ MFH_DEV mfh_u64 f64_reg(const mfh_u32* w, int k)
     else return f64_bits_of_f32(mfh_bits(decode_reg<IN>(w, k)));          // f32, f16, bf16
 }
 
-// Element i from memory (tails, misaligned buffers).
+// Element i from memory (tails).
 template <int IN>
 MFH_DEV mfh_u64 f64_at(const void* in, mfh_i64 i)
 {
@@ -949,32 +863,31 @@ MFH_DEV mfh_u64 f64_at(const void* in, mfh_i64 i)
 
 // Item = 2 elements -> one 16-byte store; the item's 2 * size source bytes
 // (one byte for two Int4 nibbles) are one load.  Elements past the last whole
-// item, and every element when a buffer is not aligned, run the element loop.
+// item run the element loop.
 template <int IN, int BS>
-__global__ __launch_bounds__(BS) void k_widen_f64(const void* __restrict__ in, void* __restrict__ out, mfh_i64 n,
-                                                      int vec_ok)
+__global__ __launch_bounds__(BS) void k_widen_f64(const void* __restrict__ in, void* __restrict__ out, mfh_i64 n)
 {
     constexpr int S = IN == kF8E4M3 || IN == kF8E5M2 ? 1 : IN == kInt4 ? 0 : size_of<IN>();
     const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
-    const mfh_i64 nitems = vec_ok ? n / 2 : 0;
-    u32x4* dst = reinterpret_cast<u32x4*>(out);
+    const mfh_i64 nitems = n / 2;
+    u32x4_any* dst = reinterpret_cast<u32x4_any*>(out);
     for (mfh_i64 v = (mfh_i64)blockIdx.x * BS + threadIdx.x; v < nitems; v += stride) {
         mfh_u32 w[4] = {0u, 0u, 0u, 0u};
         if constexpr (S == 8) {
-            const u32x4 x = load_nt(reinterpret_cast<const u32x4*>(in) + v);
+            const u32x4 x = load16<true>(static_cast<const u32x4_any*>(in) + v);
             w[0] = x[0], w[1] = x[1], w[2] = x[2], w[3] = x[3];
         } else if constexpr (S == 4) {
-            const u32x2 x = reinterpret_cast<const u32x2*>(in)[v];
+            const u32x2 x = load8<false>(static_cast<const u32x2_any*>(in) + v);
             w[0] = x[0], w[1] = x[1];
         } else if constexpr (S == 2) {
-            w[0] = reinterpret_cast<const mfh_u32*>(in)[v];
+            w[0] = load4(static_cast<const u32_any*>(in) + v);
         } else if constexpr (S == 1) {
-            w[0] = reinterpret_cast<const mfh_u16*>(in)[v];
+            w[0] = load2(static_cast<const u16_any*>(in) + v);
         } else {
             w[0] = static_cast<const mfh_u8*>(in)[v];  // Int4: two nibbles
         }
         const mfh_u64 a = f64_reg<IN>(w, 0), b = f64_reg<IN>(w, 1);
-        store_nt(&dst[v], u32x4{(mfh_u32)a, (mfh_u32)(a >> 32), (mfh_u32)b, (mfh_u32)(b >> 32)});
+        store16(&dst[v], u32x4{(mfh_u32)a, (mfh_u32)(a >> 32), (mfh_u32)b, (mfh_u32)(b >> 32)});
     }
     for (mfh_i64 i = nitems * 2 + (mfh_i64)blockIdx.x * BS + threadIdx.x; i < n; i += stride)
         static_cast<mfh_u64*>(out)[i] = f64_at<IN>(in, i);
@@ -985,13 +898,12 @@ int launch_widen_f64(const Device* dev, void* out, const void* in, int in_dt, in
     const int size = in_dt == kF8E4M3 || in_dt == kF8E5M2 ? 1 : in_dt == kInt4 ? 0 : dtype_size(in_dt);
     if (size == 0 && in_dt != kInt4)
         return fail(MFH_ERR_DTYPE_UNSUPPORTED, "mfh_convert: input dtype %s is not supported", dtype_name(in_dt));
-    const int vec_ok = aligned16(out) && aligned(in, (unsigned)std::max(1, 2 * size)) && n >= 2;
     return with_block(cast_threads(in_dt, 8), [&](auto block) {
         constexpr int BS = decltype(block)::value;
-        const unsigned grid = vec_ok ? grid_for(n / 2, dev, Kern::kConvert, 1, BS) : grid_for(n, dev, Kern::kConvert, 1, BS);
+        const unsigned grid = grid_for(std::max<int64_t>(n / 2, 1), dev, Kern::kConvert, 1, BS);
         switch (in_dt) {
 #define MFH_WIDEN_CASE(DT) \
-    case DT: k_widen_f64<DT, BS><<<grid, BS, 0, stream>>>(in, out, n, vec_ok); break;
+    case DT: k_widen_f64<DT, BS><<<grid, BS, 0, stream>>>(in, out, n); break;
             MFH_WIDEN_CASE(kFloat64)
             MFH_WIDEN_CASE(kFloat32)
             MFH_WIDEN_CASE(kFloat16)
@@ -1034,16 +946,15 @@ struct Fp8Launch {
                    hipStream_t stream)
     {
         constexpr int codes = OUT == kFloat32 ? 4 : 8;
-        int vec_ok = aligned(in, codes) && aligned16(out);
-        int64_t items = vec_ok ? std::max<int64_t>(n / codes, 1) : n;
+        const int64_t items = std::max<int64_t>(n / codes, 1);
         const mfh_u8* src = static_cast<const mfh_u8*>(in);
         const int u = items_per_thread(Kern::kFp8);
         return with_block(threads_per_block(Kern::kFp8), [&](auto block) {
             constexpr int BS = decltype(block)::value;
             const unsigned grid = grid_for(items, dev, Kern::kFp8, u, BS);
-            if (u == 4) k_dequant_fp8<OUT, 4, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt, vec_ok);
-            else if (u == 2) k_dequant_fp8<OUT, 2, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt, vec_ok);
-            else k_dequant_fp8<OUT, 1, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt, vec_ok);
+            if (u == 4) k_dequant_fp8<OUT, 4, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
+            else if (u == 2) k_dequant_fp8<OUT, 2, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
+            else k_dequant_fp8<OUT, 1, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
             return launch_status("k_dequant_fp8");
         });
     }
@@ -1064,7 +975,7 @@ struct Int4Launch {
     {
         constexpr int elems = OUT == kFloat32 ? 4 : 8;
         int shift = log2_exact(group);
-        int vec_ok = aligned(packed, elems / 2) && aligned16(out) && shift >= 0 && group >= elems;
+        int vec_ok = shift >= 0 && group >= elems;
         int64_t items = vec_ok ? std::max<int64_t>(n / elems, 1) : n;
         const int u = items_per_thread(Kern::kInt4);
         const mfh_u8* p = static_cast<const mfh_u8*>(packed);
@@ -1104,87 +1015,58 @@ struct ConvertLaunch {
     static int run_bs(const Device* dev, void* out, const void* in, int in_dt, int64_t n, hipStream_t stream)
     {
         constexpr int per = OUT == kFloat32 ? 4 : 8;
-        if ((in_dt == kBFloat16 || in_dt == kFloat16) && aligned(in, per * 2) && aligned16(out) && n % per == 0) {
-            int64_t nitems = n / per;
-            // one item per thread unless the launch config sets two: the
-            // widening to f32 ran 1% slower with two
-            const int u = items_per_thread(Kern::kConvert) >= 2 ? 2 : 1;
-            unsigned grid = grid_for(nitems, dev, Kern::kConvert, u, BS);
-            if (in_dt == kBFloat16 && u == 2) k_convert16_vec<kBFloat16, OUT, BS, 2><<<grid, BS, 0, stream>>>(in, out, nitems);
-            else if (in_dt == kBFloat16) k_convert16_vec<kBFloat16, OUT, BS, 1><<<grid, BS, 0, stream>>>(in, out, nitems);
-            else if (u == 2) k_convert16_vec<kFloat16, OUT, BS, 2><<<grid, BS, 0, stream>>>(in, out, nitems);
-            else k_convert16_vec<kFloat16, OUT, BS, 1><<<grid, BS, 0, stream>>>(in, out, nitems);
-            return launch_status("k_convert16_vec");
-        }
-        {
-            // 8-byte sources, and 4-byte integers to 16-bit: one 16-byte
-            // source piece per lane
-            const int sz = dtype_size(in_dt);
-            const bool narrow = in_dt == kFloat64 || in_dt == kInt64 || in_dt == kUint64 ||
-                                (OUT != kFloat32 && (in_dt == kInt32 || in_dt == kUint32));
-            const unsigned out_bytes = (unsigned)(16 / std::max(sz, 1) * size_of<OUT>());
-            if (narrow && aligned16(in) && aligned(out, out_bytes)) {
-                const unsigned grid = grid_for(std::max<int64_t>(n / (16 / sz), 1), dev, Kern::kConvert, 1, BS);
-                const u32x4* src = static_cast<const u32x4*>(in);
-                switch (in_dt) {
-                case kFloat64: k_narrow_vec<kFloat64, OUT, BS><<<grid, BS, 0, stream>>>(src, out, n); break;
-                case kInt64: k_narrow_vec<kInt64, OUT, BS><<<grid, BS, 0, stream>>>(src, out, n); break;
-                case kUint64: k_narrow_vec<kUint64, OUT, BS><<<grid, BS, 0, stream>>>(src, out, n); break;
-                default:
-                    if constexpr (OUT != kFloat32) {
-                        if (in_dt == kInt32) k_narrow_vec<kInt32, OUT, BS><<<grid, BS, 0, stream>>>(src, out, n);
-                        else k_narrow_vec<kUint32, OUT, BS><<<grid, BS, 0, stream>>>(src, out, n);
-                    }
-                    break;
-                }
-                return launch_status("k_narrow_vec");
-            }
-        }
-        if constexpr (OUT != kFloat32) {
-            if (in_dt == kFloat32 && aligned16(in) && aligned(out, 8) && n % 4 == 0) {
-                int64_t nitems = n / 4;
-                k_narrow_f32_vec<OUT, BS><<<grid_for(nitems, dev, Kern::kConvert, 1, BS), BS, 0, stream>>>(
-                    static_cast<const u32x4*>(in), static_cast<u32x2*>(out), nitems);
-                return launch_status("k_narrow_f32_vec");
-            }
-        }
-        // every other source: whole 16-byte output items when both buffers
-        // are aligned for them, else the element loop (256 threads)
         const int src_size = dtype_size(in_dt);
-        const bool vec = src_size > 0 && aligned(in, (unsigned)std::min(per * src_size, 16)) && aligned16(out);
+        // sources wider than the output: one 16-byte source piece per lane
+        if (src_size > (int)size_of<OUT>()) {
+            const unsigned grid = grid_for(std::max<int64_t>(n / (16 / src_size), 1), dev, Kern::kConvert, 1, BS);
+            switch (in_dt) {
+            case kFloat64: k_narrow_vec<kFloat64, OUT, BS><<<grid, BS, 0, stream>>>(in, out, n); break;
+            case kInt64: k_narrow_vec<kInt64, OUT, BS><<<grid, BS, 0, stream>>>(in, out, n); break;
+            case kUint64: k_narrow_vec<kUint64, OUT, BS><<<grid, BS, 0, stream>>>(in, out, n); break;
+            default:
+                if constexpr (OUT != kFloat32) {
+                    if (in_dt == kFloat32) k_narrow_vec<kFloat32, OUT, BS><<<grid, BS, 0, stream>>>(in, out, n);
+                    else if (in_dt == kInt32) k_narrow_vec<kInt32, OUT, BS><<<grid, BS, 0, stream>>>(in, out, n);
+                    else k_narrow_vec<kUint32, OUT, BS><<<grid, BS, 0, stream>>>(in, out, n);
+                }
+                break;
+            }
+            return launch_status("k_narrow_vec");
+        }
         // items per thread: two where the output is four times the source
-        // (int8 -> f32 +14%), one elsewhere (same-width copies lose 2-3%
-        // with two, 2x widening gains nothing), unless the launch config
-        // sets them
+        // (int8 -> f32 +14%), one elsewhere (same-width copies and 2x
+        // widening lose 1-3% with two), unless the launch config sets them
         const int set_u = items_per_thread(Kern::kConvert);
         const int u = set_u > 0 ? (set_u >= 2 ? 2 : 1) : (size_of<OUT>() >= 4 * src_size ? 2 : 1);
-        const unsigned grid = vec ? grid_for(std::max<int64_t>(n / per, 1), dev, Kern::kConvert, u, BS)
-                                  : grid_for(n, dev, Kern::kConvert);
+        const unsigned grid = grid_for(std::max<int64_t>(n / per, 1), dev, Kern::kConvert, u, BS);
+        // as wide as the output or narrower: whole 16-byte output items
         switch (in_dt) {
 #define MFH_CONVERT_CASE(DT)                                                                  \
     case DT:                                                                              \
-        if (vec && u == 2) k_convert_vec<DT, OUT, BS, 2><<<grid, BS, 0, stream>>>(in, out, n); \
-        else if (vec) k_convert_vec<DT, OUT, BS, 1><<<grid, BS, 0, stream>>>(in, out, n); \
-        else k_convert<DT, OUT><<<grid, kBlock, 0, stream>>>(in, out, n);                 \
+        if (u == 2) k_convert_vec<DT, OUT, BS, 2><<<grid, BS, 0, stream>>>(in, out, n);       \
+        else k_convert_vec<DT, OUT, BS, 1><<<grid, BS, 0, stream>>>(in, out, n);              \
         break;
-        MFH_CONVERT_CASE(kFloat64)
-        MFH_CONVERT_CASE(kFloat32)
         MFH_CONVERT_CASE(kFloat16)
         MFH_CONVERT_CASE(kBFloat16)
-        MFH_CONVERT_CASE(kInt64)
-        MFH_CONVERT_CASE(kInt32)
         MFH_CONVERT_CASE(kInt16)
         MFH_CONVERT_CASE(kInt8)
-        MFH_CONVERT_CASE(kUint64)
-        MFH_CONVERT_CASE(kUint32)
         MFH_CONVERT_CASE(kUint16)
         MFH_CONVERT_CASE(kUint8)
+        case kFloat32: case kInt32: case kUint32:
+            if constexpr (OUT == kFloat32) {
+                switch (in_dt) {
+                MFH_CONVERT_CASE(kFloat32)
+                MFH_CONVERT_CASE(kInt32)
+                MFH_CONVERT_CASE(kUint32)
+                }
+            }
+            break;
 #undef MFH_CONVERT_CASE
         default:
             return fail(MFH_ERR_DTYPE_UNSUPPORTED, "mfh_convert: input dtype %s is not supported",
                         dtype_name(in_dt));
         }
-        return launch_status("k_convert");
+        return launch_status("k_convert_vec");
     }
 };
 

@@ -21,6 +21,15 @@ namespace mfh {
 typedef mfh_u32 u32x4 __attribute__((ext_vector_type(4)));
 typedef mfh_u32 u32x2 __attribute__((ext_vector_type(2)));
 
+// The same values in memory at any byte address.  Global loads and stores of
+// 2 to 16 bytes work at any alignment on gfx950 (one instruction, as for an
+// aligned address), so row slices, odd widths and tensors inside a file image
+// take the kernels' whole-item paths like any other buffer.
+typedef mfh_u32 u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef mfh_u32 u32x2_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef mfh_u32 u32_any __attribute__((aligned(1)));
+typedef mfh_u16 u16_any __attribute__((aligned(1)));
+
 constexpr int kBlock = 256;  // 4 wave64 per workgroup: families without a size setting
 
 // Grid for `items` work items of `per_thread` items each in workgroups of
@@ -60,6 +69,36 @@ int with_block_to_512(int threads, F&& f)
 
 int launch_status(const char* what);
 
+// Loads of 16, 8, 4 and 2 bytes, non-temporal (global_load ... nt) where NT.
+// Non-temporal loads pay where a kernel reads at least as many bytes as it
+// writes (+4% on a 1:1 stream and +8% on 2:1), and for the FP8 dequant (+0.6%
+// with its codes coming from HBM); the Int4 dequant (-0.8%) and the widening
+// casts keep plain loads.
+template <bool NT>
+__device__ inline u32x4 load16(const void* p)
+{
+    const u32x4_any* q = static_cast<const u32x4_any*>(p);
+    if constexpr (NT) return __builtin_nontemporal_load(q);
+    else return *q;
+}
+
+template <bool NT>
+__device__ inline u32x2 load8(const void* p)
+{
+    const u32x2_any* q = static_cast<const u32x2_any*>(p);
+    if constexpr (NT) return __builtin_nontemporal_load(q);
+    else return *q;
+}
+
+__device__ inline mfh_u32 load4(const void* p) { return *static_cast<const u32_any*>(p); }
+__device__ inline mfh_u32 load2(const void* p) { return *static_cast<const u16_any*>(p); }
+
+// Streaming stores (global_store ... nt).
+__device__ inline void store16(void* p, u32x4 v) { __builtin_nontemporal_store(v, static_cast<u32x4_any*>(p)); }
+__device__ inline void store8(void* p, u32x2 v) { __builtin_nontemporal_store(v, static_cast<u32x2_any*>(p)); }
+__device__ inline void store4(void* p, mfh_u32 v) { __builtin_nontemporal_store(v, static_cast<u32_any*>(p)); }
+__device__ inline void store2(void* p, mfh_u32 v) { __builtin_nontemporal_store((mfh_u16)v, static_cast<u16_any*>(p)); }
+
 // Streaming 16-byte stores of a chunk: buffer stores with the non-temporal
 // (nt) and sc1 cache-policy bits, addressed from the chunk's first item (the
 // base is uniform across the block, so the descriptor lives in SGPRs).  On
@@ -67,40 +106,29 @@ int launch_status(const char* what);
 // (1:2 read:write) at 6.1-6.2 TB/s and the Int4 dequant (1:4) at 6.0-6.1,
 // against 5.8 and 5.5 with plain stores; nt alone is 1-2% slower, sc1 alone
 // 4-6%.  The descriptor's record count is the chunk's remaining bytes, so the
-// hardware drops anything past the end of the output.
+// hardware drops anything past the end of the output.  A base that is not
+// dword-aligned takes global stores (nt), which any address allows.
 struct StreamOut {
+    char* at;
+    int64_t left;
+    bool dwords;
     __amdgpu_buffer_rsrc_t rsrc;
-    __device__ StreamOut(u32x4* base, int64_t items_left)
-        : rsrc(__builtin_amdgcn_make_buffer_rsrc(
+    __device__ StreamOut(char* base, int64_t items_left)
+        : at(base), left(items_left), dwords((reinterpret_cast<uintptr_t>(base) & 3u) == 0),
+          rsrc(__builtin_amdgcn_make_buffer_rsrc(
               base, 0, (int)std::min<int64_t>(items_left * 16, 0x7fffffff), kBufferConfig))
     {
     }
     __device__ void store(int item, u32x4 v) const
     {
-        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, item * 16, 0, kCachePolicy);
+        if (dwords) __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, item * 16, 0, kCachePolicy);
+        else if (item < left) store16(at + (int64_t)item * 16, v);
     }
     // Word 3 of a raw (untyped) gfx9 buffer descriptor.
     static constexpr int kBufferConfig = 0x00020000;
     // gfx950 buffer cache policy: bit 1 nt, bit 4 sc1.
     static constexpr int kCachePolicy = 2 | 16;
 };
-
-// Streaming store through a plain address (global_store ... nt).
-template <typename T>
-__device__ inline void store_nt(T* p, T v)
-{
-    __builtin_nontemporal_store(v, p);
-}
-
-// Streaming load (global_load ... nt).  Used where a kernel reads at least as
-// many bytes as it writes (non-temporal loads measured +4% on a 1:1 stream
-// and +8% on 2:1), and by the FP8 dequant (+0.6% with its codes coming from
-// HBM); the Int4 dequant (-0.8%) and the widening casts keep plain loads.
-template <typename T>
-__device__ inline T load_nt(const T* p)
-{
-    return __builtin_nontemporal_load(p);
-}
 
 }  // namespace mfh
 
