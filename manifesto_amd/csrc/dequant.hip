@@ -157,65 +157,132 @@ MFH_DEV float load_scale(const void* scales, mfh_i64 g)
 
 MFH_DEV bool finite_f32(float f) { return (mfh_bits(f) & 0x7f800000u) != 0x7f800000u; }
 
-// Item = 8 nibbles (4 packed bytes, 16-bit output) or 4 nibbles (2 bytes,
-// f32 output) sharing one scale -> one 16-byte store.  The vector path needs
-// a power-of-two group (2^group_shift >= the item); other groups run the
-// element loop.  A block of BS threads takes chunks of BS * U consecutive
-// items (thread t holds items t, t + BS, ...), one-shot by default, with
-// streaming stores (StreamOut) addressed from the chunk's first item.  The
-// chunks are contiguous, as FP8's: a grid-stride loop whose U items per
-// thread sat a grid apart made the launch sweep U regions of the tensor at
-// once, which on this write-heavy mix ran 5.2 against 6.2 TB/s once the
-// nibbles no longer fit in the Infinity Cache.
-template <int OUT, int SDT, int U, int BS>
-__global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ packed,
-                                                         const void* __restrict__ scales,
-                                                         void* __restrict__ out, mfh_i64 n,
-                                                         mfh_i64 group, int group_shift, int vec_ok)
+// A group size as the kernels divide by it.
+struct Int4Group {
+    mfh_i64 size;
+    int shift;       // log2(size), or -1
+    mfh_u32 step;    // elements per step of an item's group number: size, or kWide for larger groups
+    mfh_u32 mul;     // 2^32 / step, rounded up: x / step = mul_hi(x, mul)
+    double inverse;  // 1 / size
+    static constexpr mfh_u32 kWide = 1u << 16, kWideFrom = 1u << 15;
+};
+
+// The scales of a chunk's items.  Element e0 of the chunk's first item lies in
+// group g0, r elements into it; both are uniform across the workgroup.  With
+// item j starting x = r + j elements further on, x / size groups past g0:
+//
+// ANY = false, a power of two of at least an item's elements: x >> shift, and
+// an item never leaves its group.  A chunk spans at most 2^14 elements, so
+// larger groups take the shift 20 and r' = 2^20 - (elements from e0 to the
+// group's end), or 0 when that end lies past the chunk, which give the same 0
+// or 1: every item runs one 32-bit add and shift.
+//
+// ANY = true, any other size of at least an item's elements: an item can hold
+// the end of one group and the start of the next, and reads both scales.  The
+// quotient for e0 by the rounded inverse is at most one off.  For groups up
+// to 2^15, x stays below 2^16, where the multiplication by 2^32 / step
+// rounded up divides exactly; a larger group takes steps of 2^16 and r' =
+// 2^16 - (elements to the group's end), as above.
+template <int ELEMS, bool ANY>
+struct Int4Scales {
+    mfh_i64 g0;
+    mfh_u32 x0, step, mul;
+    int shift;
+
+    __device__ Int4Scales(const Int4Group& group, mfh_i64 e0)
+    {
+        if constexpr (!ANY) {
+            g0 = e0 >> group.shift;
+            const mfh_u64 r = (mfh_u64)(e0 - (g0 << group.shift));
+            const bool small_group = group.shift <= 20;
+            const mfh_u64 to_next = (1ull << min(group.shift, 62)) - r;
+            x0 = small_group ? (mfh_u32)r : to_next >= (1u << 20) ? 0u : (1u << 20) - (mfh_u32)to_next;
+            shift = small_group ? group.shift : 20;
+        } else {
+            const mfh_u64 q = (mfh_u64)((double)e0 * group.inverse);
+            g0 = (mfh_i64)((mfh_u64)__builtin_amdgcn_readfirstlane((mfh_u32)(q >> 32)) << 32 |
+                           (mfh_u32)__builtin_amdgcn_readfirstlane((mfh_u32)q));
+            mfh_i64 r = e0 - g0 * group.size;
+            if (r < 0) g0--, r += group.size;
+            if (r >= group.size) g0++, r -= group.size;
+            const mfh_i64 to_next = group.size - r;
+            step = group.step;
+            mul = group.mul;
+            x0 = step != Int4Group::kWide ? (mfh_u32)r
+                 : to_next >= (mfh_i64)Int4Group::kWide ? 0u : Int4Group::kWide - (mfh_u32)to_next;
+        }
+    }
+
+    // The group (past g0) of the item that starts `at` elements into the
+    // chunk, and how many of its elements lie in it (ANY; else all).
+    __device__ mfh_u32 group_of(mfh_u32 at, int* own) const
+    {
+        const mfh_u32 x = x0 + at;
+        if constexpr (!ANY) {
+            *own = ELEMS;
+            return x >> shift;
+        } else {
+            const mfh_u32 g = __umulhi(x, mul);
+            *own = (int)((g + 1) * step - x);
+            return g;
+        }
+    }
+};
+
+// Item = 8 nibbles (4 packed bytes, 16-bit output) or 4 nibbles (2 bytes, f32
+// output) -> one 16-byte store.  Groups smaller than an item run the element
+// loop.  A block of BS threads takes chunks of BS * U consecutive items
+// (thread t holds items t, t + BS, ...), one-shot by default, with streaming
+// stores (StreamOut) addressed from the chunk's first item.  The chunks are
+// contiguous, as FP8's: a grid-stride loop whose U items per thread sat a
+// grid apart made the launch sweep U regions of the tensor at once, which on
+// this write-heavy mix ran 5.2 against 6.2 TB/s once the nibbles no longer
+// fit in the Infinity Cache.  bf16 from [4096, 14336] with an f32 scale per
+// row, MI355X: 22.1 us, against 110.8 by the element loop (2-byte
+// stores, a 64-bit division per element), which every group that is not a
+// power of two took; with groups of 128 the shift runs 21.5 us where the
+// multiplication ran 21.6-21.9.
+template <int OUT, int SDT, int U, int BS, bool ANY>
+MFH_DEV void dequant_int4(const mfh_u8* __restrict__ packed, const void* __restrict__ scales,
+                          void* __restrict__ out, mfh_i64 n, const Int4Group& group, bool vec_ok)
 {
     constexpr int kElems = OUT == kFloat32 ? 4 : 8;
     constexpr mfh_i64 kChunk = (mfh_i64)BS * U;
+    static_assert(kChunk * kElems <= (1 << 14), "a chunk spans at most 2^14 elements");
     const mfh_i64 nitems = vec_ok ? n / kElems : 0;
     const mfh_i64 nchunks = (nitems + kChunk - 1) / kChunk;
     const int t = (int)threadIdx.x;
     for (mfh_i64 c = blockIdx.x; c < nchunks; c += gridDim.x) {
         const mfh_i64 first = c * kChunk;
-        // Lane addresses are 32-bit offsets from uniform bases: the chunk's
-        // first packed item and its first item's group scale (element e0,
-        // group g0, e0 = g0 * group + r).  Items past the end load the last
-        // item instead of branching: a guarded load made the compiler wait
-        // for each scale inside its branch, one round trip per item, before
-        // issuing the next item's loads (5.3 against 6.2 TB/s).
+        // Lane addresses are 32-bit offsets from uniform bases, the chunk's
+        // first packed item and its first item's group scale.  Items past the
+        // end load the last item instead of branching: a guarded load made
+        // the compiler wait for each scale inside its branch, one round trip
+        // per item, before issuing the next item's loads (5.3 against 6.2
+        // TB/s).
         const int last = (int)min<mfh_i64>(kChunk, nitems - first) - 1;
-        const mfh_i64 e0 = first * kElems;
-        const mfh_i64 g0 = e0 >> group_shift;
-        const mfh_u64 r = (mfh_u64)(e0 - (g0 << group_shift));
         constexpr mfh_u32 kItemBytes = kElems / 2, kScaleBytes = SDT == kFloat32 ? 4 : 2;
         const char* items = reinterpret_cast<const char*>(packed) + first * kItemBytes;
-        const char* group0 = static_cast<const char*>(scales) + g0 * kScaleBytes;
-        // The item's group relative to g0 is (r + j kElems) >> group_shift.
-        // A chunk spans fewer than 2^20 elements, so for larger groups the
-        // same formula with shift 20 and r' = 2^20 - (elements from e0 to
-        // the next group boundary), or 0 when that boundary lies past the
-        // chunk, gives the same 0 or 1: every item runs one 32-bit add and
-        // shift.
-        static_assert(kChunk * kElems < (1 << 20), "a chunk spans fewer than 2^20 elements");
-        const bool small_group = group_shift <= 20;
-        const mfh_u64 to_next = (1ull << min(group_shift, 62)) - r;
-        const mfh_u32 gr = small_group ? (mfh_u32)r : to_next >= (1u << 20) ? 0u : (1u << 20) - (mfh_u32)to_next;
-        const int gs = small_group ? group_shift : 20;
-        mfh_u32 w[U], sb[U];
+        const Int4Scales<kElems, ANY> map(group, first * kElems);
+        const char* group0 = static_cast<const char*>(scales) + map.g0 * kScaleBytes;
+        mfh_u32 w[U], sb[U], sb1[U];
+        int own[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const mfh_u32 j = (mfh_u32)min(u * BS + t, last);
             if constexpr (kElems == 8) w[u] = load4(items + j * kItemBytes);
             else w[u] = load2(items + j * kItemBytes);
-            sb[u] = scale_bits<SDT>(group0 + ((gr + j * kElems) >> gs) * kScaleBytes, 0);
+            const mfh_u32 g = map.group_of(j * kElems, &own[u]);
+            sb[u] = scale_bits<SDT>(group0 + g * kScaleBytes, 0);
+            if constexpr (ANY) sb1[u] = scale_bits<SDT>(group0 + (own[u] < kElems ? g + 1 : g) * kScaleBytes, 0);
         }
         __builtin_amdgcn_sched_barrier(0);  // every load of the chunk ahead of the first wait
-        float s[U];
+        float s[U], s1[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) s[u] = scale_value<SDT>(sb[u]);
+        for (int u = 0; u < U; u++) {
+            s[u] = scale_value<SDT>(sb[u]);
+            s1[u] = ANY ? scale_value<SDT>(sb1[u]) : s[u];
+        }
         // The buffer descriptor ends at the last item: stores past it are dropped.
         const StreamOut dst(static_cast<char*>(out) + first * 16, nitems - first);
 #pragma unroll
@@ -223,10 +290,12 @@ __global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ 
             const int j = u * BS + t;
             float f[kElems];
 #pragma unroll
-            for (int k = 0; k < kElems; k++) f[k] = (float)mfh_int4_at(w[u], k) * s[u];
-            if (!finite_f32(s[u])) {  // Inf/NaN scale: apply the explicit NaN rules (rare)
+            for (int k = 0; k < kElems; k++)
+                f[k] = (float)mfh_int4_at(w[u], k) * (ANY && k >= own[u] ? s1[u] : s[u]);
+            if (!finite_f32(s[u]) || (ANY && !finite_f32(s1[u]))) {  // Inf/NaN scale: the explicit NaN rules (rare)
 #pragma unroll
-                for (int k = 0; k < kElems; k++) f[k] = mfh_scale_mul((float)mfh_int4_at(w[u], k), s[u]);
+                for (int k = 0; k < kElems; k++)
+                    f[k] = mfh_scale_mul((float)mfh_int4_at(w[u], k), ANY && k >= own[u] ? s1[u] : s[u]);
             }
             if constexpr (OUT == kFloat32)
                 dst.store(j, u32x4{mfh_bits(f[0]), mfh_bits(f[1]), mfh_bits(f[2]), mfh_bits(f[3])});
@@ -239,9 +308,30 @@ __global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ 
     for (mfh_i64 i = nitems * kElems + (mfh_i64)blockIdx.x * BS + threadIdx.x; i < n; i += stride) {
         mfh_u32 byte = packed[i >> 1];
         float q = (float)mfh_int4_at(byte, (mfh_u32)(i & 1));
-        float s = load_scale<SDT>(scales, i / group);
+        float s = load_scale<SDT>(scales, i / group.size);
         store_one<OUT>(out, i, encode_one<OUT>(mfh_scale_mul(q, s)));
     }
+}
+
+// The two kernels take just the arguments they use: gfx950 preloads the first
+// 14 dwords into SGPRs, and the grid size that follows a longer list costs
+// every wave a scalar load ahead of its first vector load (0.5% at 147 MB).
+template <int OUT, int SDT, int U, int BS>
+__global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ packed,
+                                                         const void* __restrict__ scales,
+                                                         void* __restrict__ out, mfh_i64 n, mfh_i64 size,
+                                                         int shift, int vec_ok)
+{
+    dequant_int4<OUT, SDT, U, BS, false>(packed, scales, out, n, Int4Group{size, shift, 0u, 0u, 0.0}, vec_ok != 0);
+}
+
+template <int OUT, int SDT, int U, int BS>
+__global__ __launch_bounds__(BS) void k_dequant_int4_any(const mfh_u8* __restrict__ packed,
+                                                             const void* __restrict__ scales,
+                                                             void* __restrict__ out, mfh_i64 n, mfh_u32 step,
+                                                             mfh_u32 mul, double inverse, mfh_i64 size)
+{
+    dequant_int4<OUT, SDT, U, BS, true>(packed, scales, out, n, Int4Group{size, -1, step, mul, inverse}, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -960,44 +1050,57 @@ struct Fp8Launch {
     }
 };
 
-int log2_exact(int64_t g)
-{
-    if (g <= 0 || (g & (g - 1)) != 0) return -1;
-    int s = 0;
-    while ((int64_t(1) << s) < g) s++;
-    return s;
-}
-
 template <int OUT>
 struct Int4Launch {
     static int run(const Device* dev, void* out, const void* packed, int64_t n, const void* scales,
-                   int scale_dt, int64_t group, hipStream_t stream)
+                   int scale_dt, int64_t size, hipStream_t stream)
     {
         constexpr int elems = OUT == kFloat32 ? 4 : 8;
-        int shift = log2_exact(group);
-        int vec_ok = shift >= 0 && group >= elems;
-        int64_t items = vec_ok ? std::max<int64_t>(n / elems, 1) : n;
+        Int4Group group;
+        group.size = size;
+        group.inverse = 1.0 / (double)size;
+        group.shift = size & (size - 1) ? -1 : __builtin_ctzll((uint64_t)size);
+        group.step = size > (int64_t)Int4Group::kWideFrom ? Int4Group::kWide : (mfh_u32)size;
+        // (step 1, an element-loop group, has no 32-bit multiplier and needs none)
+        const uint64_t range = uint64_t(1) << 32;
+        group.mul = (mfh_u32)(range / group.step + (range % group.step != 0));
+        const int vec_ok = size >= elems;
+        const bool any = vec_ok && group.shift < 0;
+        const int64_t items = vec_ok ? std::max<int64_t>(n / elems, 1) : n;
         const int u = items_per_thread(Kern::kInt4);
         const mfh_u8* p = static_cast<const mfh_u8*>(packed);
         return with_block_to_512(threads_per_block(Kern::kInt4), [&](auto block) {
             constexpr int BS = decltype(block)::value;
             const unsigned grid = grid_for(items, dev, Kern::kInt4, u, BS);
-            if (u == 4) launch<4, BS>(grid, p, scales, scale_dt, out, n, group, shift, vec_ok, stream);
-            else if (u == 2) launch<2, BS>(grid, p, scales, scale_dt, out, n, group, shift, vec_ok, stream);
-            else launch<1, BS>(grid, p, scales, scale_dt, out, n, group, shift, vec_ok, stream);
+            if (u == 4) launch<4, BS>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
+            else if (u == 2) launch<2, BS>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
+            else launch<1, BS>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
             return launch_status("k_dequant_int4");
         });
     }
 
     template <int U, int BS>
     static void launch(unsigned grid, const mfh_u8* p, const void* scales, int scale_dt, void* out, int64_t n,
-                       int64_t group, int shift, int vec_ok, hipStream_t stream)
+                       const Int4Group& group, int vec_ok, bool any, hipStream_t stream)
     {
         switch (scale_dt) {
-        case kFloat32: k_dequant_int4<OUT, kFloat32, U, BS><<<grid, BS, 0, stream>>>(p, scales, out, n, group, shift, vec_ok); break;
-        case kFloat16: k_dequant_int4<OUT, kFloat16, U, BS><<<grid, BS, 0, stream>>>(p, scales, out, n, group, shift, vec_ok); break;
-        case kBFloat16: k_dequant_int4<OUT, kBFloat16, U, BS><<<grid, BS, 0, stream>>>(p, scales, out, n, group, shift, vec_ok); break;
-        default: k_dequant_int4<OUT, kInvalid, U, BS><<<grid, BS, 0, stream>>>(p, scales, out, n, group, shift, vec_ok); break;
+#define MFH_INT4_CASE(DT)                                                                                           \
+    case DT:                                                                                                        \
+        if (any)                                                                                                    \
+            k_dequant_int4_any<OUT, DT, U, BS>                                                                      \
+                <<<grid, BS, 0, stream>>>(p, scales, out, n, group.step, group.mul, group.inverse, group.size);     \
+        else                                                                                                        \
+            k_dequant_int4<OUT, DT, U, BS>                                                                          \
+                <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift, vec_ok);                      \
+        break;
+            MFH_INT4_CASE(kFloat32)
+            MFH_INT4_CASE(kFloat16)
+            MFH_INT4_CASE(kBFloat16)
+#undef MFH_INT4_CASE
+        default:
+            k_dequant_int4<OUT, kInvalid, U, BS>
+                <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift, vec_ok);
+            break;
         }
     }
 };
