@@ -199,13 +199,13 @@ typedef struct {
 
 /* Transcendental nodes evaluated in f64 exactly as codegen/cpu.go:172-200
  * writes them (bit-identical to the reference but for f64 rounding ties).
- * Sigmoid, Silu and Gelu take f64 forms with about two thirds of the
- * reference's instructions, whose result is used where a test shows that it
- * rounds to the same f32 as the reference's value; the elements the test
- * cannot decide (about one in 2^13) are recomputed with the reference's
- * formulas.  Without it, chains that stream f32 take the same forms, and
- * chains of 16-bit operands f32 Silu and Gelu within 2 ulp and an f64
- * Sigmoid within 1. */
+ * They take f64 forms with a fraction of the reference formulas' instructions,
+ * whose result is used where a test shows that it rounds to the same f32 as
+ * the reference's value; the elements the test cannot decide (about one in
+ * 2^13, fewer for Log and Tanh) are recomputed with the reference's formulas.
+ * Without it, Exp, Log and Tanh take the same forms in every chain, and so do
+ * Sigmoid, Silu and Gelu in chains that stream f32; chains of 16-bit operands
+ * take f32 Silu and Gelu within 2 ulp and an f64 Sigmoid within 1. */
 #define MFH_FUSION_PRECISE 1u
 
 /* Sigmoid, Silu and Gelu in the fast forms of chains of 16-bit operands in

@@ -333,8 +333,9 @@ MFH_MATH double mfh_gelu_z(float c, double& den)
 // than z does.  z must round to a normal f32 of magnitude above 2^-126.
 MFH_MATH bool mfh_near_f32_midpoint(double z, unsigned margin)
 {
-    const unsigned low = (unsigned)mfh_low_int(z) & 0x1fffffffu;
-    return low - (0x10000000u - margin) < 2u * margin;
+    // the 29 bits sit on top of the word, so that the subtraction wraps with them
+    const unsigned low = (unsigned)mfh_low_int(z) << 3;
+    return low - ((0x10000000u - margin) << 3) < margin << 4;
 }
 
 // False for NaN, infinities, zeros, subnormals and 2^-126 itself, which an
@@ -381,6 +382,120 @@ MFH_MATH float mfh_gelu_cr(float v, bool& rare)
     return r;
 }
 
+// exp, log and tanh in the same way: f64 forms close enough to the exact
+// value that the rounding test decides almost every element, in place of
+// library calls (codegen/cpu.go:177-185 evaluates math.Exp, math.Log and
+// math.Tanh in f64 and rounds once).  On MI355X, 2^24 elements: cap *
+// tanh(x / cap) over f32 27.5 us (78 with the library's f64 tanh), over bf16
+// 23 (77); log(e^x + 1) over f32 31 (60), over bf16 27 (56).  Still bound by
+// the f64 arithmetic (about 45 instructions per element for tanh), not by
+// the 19.5 and 9.7 us of the memory traffic.
+
+MFH_MATH float mfh_exp_ref(float v) { return (float)mfh_exp_f64((double)v); }
+MFH_MATH float mfh_log_ref(float v) { return (float)mfh_log_f64((double)v); }
+MFH_MATH float mfh_tanh_ref(float v) { return (float)mfh_tanh_f64((double)v); }
+
+// e^m, m in [-104, 89]: 2^t, t = m log2(e), to 2^-39.8 (as mfh_sigmoid_z).
+MFH_MATH double mfh_exp_z(float m)
+{
+    const double x = (double)m;
+    const double tk = mfh_fma(x, MFH_LOG2E_D, MFH_ROUND_INT_D);
+    const double kd = tk - MFH_ROUND_INT_D;
+    return mfh_ldexp(mfh_exp2_poly_d(mfh_fma(x, MFH_LOG2E_D, -kd)), mfh_low_int(tk));
+}
+
+// The clamp changes no result: e^v rounds to 0 below -104 (e^-104 < 2^-150)
+// and to Inf above 89, which masked elements rely on.  Flagged: NaN and the
+// subnormal results in between, besides the undecided ones.
+MFH_MATH float mfh_exp_cr(float v, bool& rare)
+{
+    const float m = mfh_med3f(v, -104.0f, 89.0f);
+    const double z = mfh_exp_z(m);
+    const float r = (float)z;
+    rare |= mfh_is_nan(v) | ((m > -104.0f) & (r <= 0x1p-126f)) | mfh_near_f32_midpoint(z, 1u << 15);
+    return r;
+}
+
+// log v for a positive normal v = 2^e m, m in [sqrt(1/2), sqrt(2)):
+// e ln2 + log m, log m = 2 atanh(s), s = (m - 1) / (m + 1), |s| < 0.1716, as
+// 2s + s^3 P(s^2) with P of degree 4 (the fit of gen_exp_poly.py, 2^-44.8
+// relative; e != 0 leaves at least 0.34 of the sum, so the relative error
+// stays below 2^-43).  m - 1 and m + 1 are exact.
+MFH_MATH double mfh_log_z(float v)
+{
+    const unsigned u = mfh_fbits(v) - 0x3f3504f3u;  // bits of sqrt(1/2)
+    const double e = (double)((int)u >> 23);
+    const double m = (double)mfh_fromfbits((u & 0x7fffffu) + 0x3f3504f3u);
+    const double s = (m - 1.0) * mfh_recip_newton(m + 1.0);
+    const double y = s * s;
+    double p = 0x1.9121bb51a0838p-3;
+    p = mfh_fma(p, y, 0x1.c62a1f8778661p-3);
+    p = mfh_fma(p, y, 0x1.24941556fb569p-2);
+    p = mfh_fma(p, y, 0x1.9999969f50b5bp-2);
+    p = mfh_fma(p, y, 0x1.555555562327bp-1);
+    return mfh_fma(e, MFH_LN2_D, mfh_fma(s * y, p, s + s));
+}
+
+// Flagged: zeros, subnormals, negatives, infinities and NaN, besides the
+// undecided ones; log 1 = 0 is exact.  The margin of 2^12 f64 ulps is at
+// least 2^-41 of the value.
+MFH_MATH float mfh_log_cr(float v, bool& rare)
+{
+    const double z = mfh_log_z(v);
+    rare |= !((v >= 0x1p-126f) & (v <= 0x1.fffffep127f)) | mfh_near_f32_midpoint(z, 1u << 12);
+    return (float)z;
+}
+
+// tanh a for a in [0, 20]: n / (n + 2), n = e^(2a) - 1 = 2^k (1 + f q(f)) - 1
+// with 2^k 2^f = e^(2a).  f q(f) = 2^f - 1 is fitted relative to n on both
+// sides (degree 9, 2^-43 by gen_exp_poly.py), so small arguments keep their
+// relative accuracy; the subtraction of 1 costs 2^-54 / n, 2^-43 at a =
+// 2^-12.
+MFH_MATH double mfh_tanh_z(float a)
+{
+    const double x = (double)a;
+    const double tk = mfh_fma(x, 2.0 * MFH_LOG2E_D, MFH_ROUND_INT_D);
+    const double kd = tk - MFH_ROUND_INT_D;
+    const double f = mfh_fma(x, 2.0 * MFH_LOG2E_D, -kd);
+    double q = 0x1.b55c9834c77e8p-24;
+    q = mfh_fma(q, f, 0x1.63e23afd28442p-20);
+    q = mfh_fma(q, f, 0x1.ffcc22651411fp-17);
+    q = mfh_fma(q, f, 0x1.43089c1a418bdp-13);
+    q = mfh_fma(q, f, 0x1.5d87fe8b53bc2p-10);
+    q = mfh_fma(q, f, 0x1.3b2ab721ae45ap-7);
+    q = mfh_fma(q, f, 0x1.c6b08d7013121p-5);
+    q = mfh_fma(q, f, 0x1.ebfbdff81d73bp-3);
+    q = mfh_fma(q, f, 0x1.62e42fefa3cb5p-1);
+    const double n = mfh_ldexp(mfh_fma(q, f, 1.0), mfh_low_int(tk)) - 1.0;
+    return n * mfh_recip_newton(n + 2.0);
+}
+
+// tanh v = v (1 - v^2 / 3 + ...) rounds to v up to 2^-12 (v^2 / 3 < 2^-25)
+// and to +-1 from 9.02 on, so neither end is flagged; NaN is.  The margin of
+// 2^13 f64 ulps is at least 2^-40 of the value.
+MFH_MATH float mfh_tanh_cr(float v, bool& rare)
+{
+    const float a = mfh_minf(mfh_absf(v), 20.0f);
+    const double z = mfh_tanh_z(a);
+    const bool self = a <= 0x1p-12f;
+    const float r = mfh_fromfbits(mfh_fbits((float)z) | (mfh_fbits(v) & 0x80000000u));
+    rare |= mfh_is_nan(v) | (!self & mfh_near_f32_midpoint(z, 1u << 13));
+    return self ? v : r;
+}
+
+// x / c for a constant c, as x times 1 / c rounded to f64: within 2^-52 of the
+// quotient, which lies at least 2^-49 from every point halfway between two
+// f32 neighbours (x and c have 24 bits), so its rounding to f32 is the
+// division's, with its zeros, infinities and NaN.  Where the quotient is
+// subnormal it can be exactly such a point: flagged.  The f32 division is
+// about 60 cycles of a wave, this form 27.
+MFH_MATH float mfh_div_const(float x, double inverse, bool& rare)
+{
+    const float r = (float)((double)x * inverse);
+    rare |= (mfh_fbits(r) << 1) - 1u < 0x01000000u;  // 0 < |r| <= 2^-126
+    return r;
+}
+
 // mfh_<name>_rare: the reference's result as a real call (MFH_RARE), which
 // the generated kernels use to recompute flagged elements: the
 // rounding-tested form above, and the reference form where that one flags the
@@ -410,6 +525,9 @@ MFH_MATH float mfh_gelu_cr(float v, bool& rare)
 MFH_RARE_FORM(sigmoid)
 MFH_RARE_FORM(silu)
 MFH_RARE_FORM(gelu)
+MFH_RARE_FORM(exp)
+MFH_RARE_FORM(log)
+MFH_RARE_FORM(tanh)
 #undef MFH_RARE_FORM
 MFH_FAST_OR_REF(mfh_sigmoid, mfh_sigmoid_fast, mfh_sigmoid_rare)
 MFH_FAST_OR_REF(mfh_silu, mfh_silu_fast, mfh_silu_rare)
@@ -420,10 +538,9 @@ MFH_FAST_OR_REF(mfh_gelu, mfh_gelu_fast, mfh_gelu_rare)
 MFH_FAST_OR_REF(mfh_sigmoid_p, mfh_sigmoid_cr, mfh_sigmoid_ref)
 MFH_FAST_OR_REF(mfh_silu_p, mfh_silu_cr, mfh_silu_ref)
 MFH_FAST_OR_REF(mfh_gelu_p, mfh_gelu_cr, mfh_gelu_ref)
+MFH_FAST_OR_REF(mfh_exp_p, mfh_exp_cr, mfh_exp_ref)
+MFH_FAST_OR_REF(mfh_log_p, mfh_log_cr, mfh_log_ref)
+MFH_FAST_OR_REF(mfh_tanh_p, mfh_tanh_cr, mfh_tanh_ref)
 #undef MFH_FAST_OR_REF
-
-MFH_MATH float mfh_exp_ref(float v) { return (float)mfh_exp_f64((double)v); }
-MFH_MATH float mfh_log_ref(float v) { return (float)mfh_log_f64((double)v); }
-MFH_MATH float mfh_tanh_ref(float v) { return (float)mfh_tanh_f64((double)v); }
 
 #endif  // MFH_DEVMATH_HPP

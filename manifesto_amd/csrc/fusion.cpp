@@ -66,6 +66,15 @@ std::string hex32(float f)
     return buf;
 }
 
+std::string hex64(double d)
+{
+    uint64_t u;
+    std::memcpy(&u, &d, 8);
+    char buf[64];
+    snprintf(buf, sizeof buf, "__builtin_bit_cast(double, 0x%016llxull)", (unsigned long long)u);
+    return buf;
+}
+
 // Pre-order list -> child links; -1 if malformed.
 int link(const std::vector<mfh_ast_node>& nodes, int idx, std::vector<int>& c0, std::vector<int>& c1)
 {
@@ -191,6 +200,10 @@ struct Emitter {
     // Set once the element's flag `qe` has been written: a fast activation or
     // a guard was emitted.
     bool flagged = false;
+    // Divisions by a constant take mfh_div_const: chains with a
+    // transcendental node, whose arithmetic outweighs their memory traffic
+    // and which carry the flag anyway.
+    bool const_div = false;
 
     std::string fresh() { return prefix + std::to_string(tmp++); }
 
@@ -208,6 +221,16 @@ struct Emitter {
         if (form == Form::kFallback) return let(fn + "_rare(" + a + ")");
         flagged = true;
         return let(fn + (form == Form::kRounded ? "_cr(" : "_fast(") + a + ", qe)");
+    }
+
+    // Exp, Log and Tanh: the rounding-tested forms in every chain.
+    std::string rounded(const char* name, const std::string& a)
+    {
+        const std::string fn = std::string("mfh_") + name;
+        if (form == Form::kPrecise) return let(fn + "_ref(" + a + ")");
+        if (form == Form::kFallback) return let(fn + "_rare(" + a + ")");
+        flagged = true;
+        return let(fn + "_cr(" + a + ", qe)");
     }
 
     // s = a + b (or a - b): the cancellation guard of node idx, if planned.
@@ -259,7 +282,16 @@ struct Emitter {
             case kNodeAdd: return guarded(idx, let(a + " + " + b), a, b);
             case kNodeSub: return guarded(idx, let(a + " - " + b), a, b);
             case kNodeMul: return let(a + " * " + b);
-            case kNodeDiv: return let(a + " / " + b);
+            case kNodeDiv: {
+                // by a constant, in a chain whose element math is what takes its time
+                const mfh_ast_node& by = nodes[c1[idx]];
+                const float c = (float)by.value;
+                if (const_div && by.type == kNodeConstant && std::isfinite(c) && c != 0.0f) {
+                    flagged = true;
+                    return let("mfh_div_const(" + a + ", " + hex64(1.0 / (double)c) + ", qe)");
+                }
+                return let(a + " / " + b);
+            }
             case kNodeMax: return let("(" + a + " > " + b + ") ? " + a + " : " + b);
             case kNodeMin: return let("(" + a + " < " + b + ") ? " + a + " : " + b);
             }
@@ -268,11 +300,11 @@ struct Emitter {
         case kNodeNeg: return let("-" + a);
         case kNodeAbs: return let("(" + a + " < 0.0f) ? -" + a + " : " + a);
         case kNodeSqrt: return let("mfh_sqrtf(" + a + ")");
-        case kNodeExp: return let("mfh_exp_ref(" + a + ")");
-        case kNodeLog: return let("mfh_log_ref(" + a + ")");
+        case kNodeExp: return rounded("exp", a);
+        case kNodeLog: return rounded("log", a);
         case kNodeReLU: return let("(" + a + " < 0.0f) ? 0.0f : " + a);
         case kNodeSigmoid: return activation("sigmoid", a);
-        case kNodeTanh: return let("mfh_tanh_ref(" + a + ")");
+        case kNodeTanh: return rounded("tanh", a);
         case kNodeSilu: return activation("silu", a);
         case kNodeGelu: return activation("gelu", a);
         case kNodeLeakyReLU: {
@@ -581,12 +613,13 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     // dispatch order).  Measured on MI355X against grid-stride loops at 4-24
     // blocks per CU: +11% on the SwiGLU chain and +9% on the f16 gelu chain;
     // a no-compute 2:1 read:write stream gains 17% the same way.  One item per
-    // thread, except where the element math is mostly f64 (Sigmoid, and the
-    // rounding-tested forms of chains that stream f32 and of
-    // MFH_FUSION_PRECISE): two items per thread give a sigmoid chain 0-3% and
-    // the precise SwiGLU chain 5.6% (the precise gelu chain -1%, within the
-    // noise of six alternating runs), while SwiGLU, Silu, add/mul chains and
-    // (since its 2^f runs on v_exp_f32) the gelu chain lose 2-6% and the
+    // thread, except where the element math is mostly f64 (Sigmoid, Exp, Log,
+    // Tanh, and the rounding-tested forms of chains that stream f32 and of
+    // MFH_FUSION_PRECISE): two items per thread give a tanh chain 4%, an exp
+    // and log chain 4% over f32 and 1% over bf16, a sigmoid chain 0-3% and the
+    // precise SwiGLU chain 5.6% (the precise gelu chain -1%, within the noise
+    // of six alternating runs).  SwiGLU, Silu, add/mul chains and (since its 2^f runs on
+    // v_exp_f32) the gelu chain over 16 bits lose 2-6% with two, and the
     // reference forms inline (MFH_FUSION_NO_ROUNDING_TEST) gain nothing.
     // Workgroups of one wave (kFusedThreads).  mfh_set_launch_config("fused",
     // ...) and mfh_set_launch_threads("fused", ...) override these.
@@ -601,7 +634,8 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     const bool rounded = precise ? (flags & MFH_FUSION_NO_ROUNDING_TEST) == 0 : streams_f32;
     bool f64_fast = false;
     for (const mfh_ast_node& node : list)
-        if (is_fast_activation(node.type) && (rounded || (!precise && node.type == kNodeSigmoid)))
+        if (is_fast_activation(node.type) ? rounded || (!precise && node.type == kNodeSigmoid)
+                                          : is_transcendental(node.type) && (rounded || !precise))
             f64_fast = true;
     const int unroll = items_per_thread(Kern::kFused) > 0 ? items_per_thread(Kern::kFused) : f64_fast ? 2 : 1;
     const int auto_bpc = kOneShotBlocksPerCu;
@@ -626,11 +660,15 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     std::vector<bool> packed16(n_inputs, false);
     for (int k = 0; k < n_inputs; k++)
         packed16[k] = inputs[k].mode != MFH_OPERAND_SCALAR && inputs[k].dtype == kFloat16;
+    bool const_div = false;
+    for (const mfh_ast_node& node : list) const_div |= is_transcendental(node.type) && main_form != Form::kPrecise;
     Emitter em{list, c0, c1, main_form, &guards};
+    em.const_div = const_div;
     const std::string result = em.emit(0);
     Emitter emf{list, c0, c1, Form::kFallback, nullptr, "f"};
     const std::string fresult = em.flagged ? emf.emit(0) : "";
     Emitter emv{list, c0, c1, main_form, &guards, "t", packed16};
+    emv.const_div = const_div;
     const std::string vresult = emv.emit(0);
     Emitter emvf{list, c0, c1, Form::kFallback, nullptr, "f", packed16};
     const std::string vfresult = emv.flagged ? emvf.emit(0) : "";

@@ -13,6 +13,12 @@ units and reduced in f64) is fitted the same way, once with f32 coefficients
 instead, which measured faster and equally accurate) and once with f64
 coefficients (degree 8, fitted in 50-digit arithmetic with mpmath; sigmoid).
 
+Two more f64 fits, by the same weighted least squares in 50 digits, serve tanh
+and log: 2^f - 1 = f q(f) of degree 9, relative to 2^f - 1 for f > 0 and to
+2^(1 + f) - 1 for f < 0 (fit_expm1_f64), and (2 atanh(s) - 2 s) / s^3 as a
+polynomial of degree 4 in s^2 for |s| <= (sqrt(2) - 1) / (sqrt(2) + 1)
+(fit_log_f64).
+
 Run: python3 gen_exp_poly.py
 """
 import math
@@ -81,6 +87,65 @@ def fit_exp2_f64(degree=8, half_width=0.5, nodes=600):
     return coef, float(mp.log(worst, 2))
 
 
+def lsq_f64(xs, basis, target, weight):
+    """Weighted least squares in mpmath arithmetic, coefficients rounded to f64."""
+    import mpmath as mp
+    n, d = len(xs), len(basis(xs[0]))
+    A, b = mp.matrix(n, d), mp.matrix(n, 1)
+    for i, x in enumerate(xs):
+        w = weight(x)
+        for j, v in enumerate(basis(x)):
+            A[i, j] = w * v
+        b[i] = w * target(x)
+    Q, R = mp.qr(A)
+    c = mp.lu_solve(R[:d, :d], (Q.T * b)[:d, 0])
+    return [float(c[j]) for j in range(d)]
+
+
+def chebyshev(a, b, n):
+    import mpmath as mp
+    return [(a + b) / 2 + (b - a) / 2 * mp.cos(mp.pi * (k + mp.mpf(0.5)) / n) for k in range(n)]
+
+
+def fit_expm1_f64(degree=9):
+    """tanh: coefficients of f q(f) and the largest weighted error."""
+    import mpmath as mp
+    mp.mp.dps = 50
+    two = mp.mpf(2)
+
+    def weight(f):
+        return 1 / (two ** f - 1) if f > 0 else 2 / (two ** (1 + f) - 1)
+
+    xs = chebyshev(mp.mpf(-0.5), mp.mpf(0.5), 400)
+    c = lsq_f64(xs, lambda f: [f ** (j + 1) for j in range(degree)], lambda f: two ** f - 1, weight)
+    worst = 0
+    for i in list(range(-2000, 0)) + list(range(1, 2001)):
+        f = mp.mpf(i) / 4000
+        acc = mp.mpf(0)
+        for cj in reversed(c):
+            acc = (acc + cj) * f
+        worst = max(worst, abs(acc - (two ** f - 1)) * weight(f))
+    return c, float(mp.log(worst, 2))
+
+
+def fit_log_f64(terms=5):
+    """log: coefficients in s^2 and the largest error relative to 2 atanh(s)."""
+    import mpmath as mp
+    mp.mp.dps = 50
+    top = ((mp.sqrt(2) - 1) / (mp.sqrt(2) + 1)) ** 2
+    c = lsq_f64(chebyshev(mp.mpf(0), top, 200), lambda y: [y ** j for j in range(terms)],
+                lambda y: (2 * mp.atanh(mp.sqrt(y)) - 2 * mp.sqrt(y)) / mp.sqrt(y) ** 3, lambda y: y)
+    worst = 0
+    for i in range(1, 2001):
+        y = top * i / 2000
+        s = mp.sqrt(y)
+        acc = mp.mpf(0)
+        for cj in reversed(c):
+            acc = acc * y + cj
+        worst = max(worst, abs((2 * s + s * y * acc) / (2 * mp.atanh(s)) - 1))
+    return c, float(mp.log(worst, 2))
+
+
 def horner_f32(coef, r):
     """Evaluates 1 + r*(c1 + r*(c2 + ...)) with f32 fma rounding."""
     r64 = r.astype(np.float64)
@@ -119,6 +184,11 @@ def main():
     for j, c in enumerate(coef64, start=1):
         print(f"2^f f64 c{j}", float.hex(c))
     print("log2 of the max relative error of 2^f in f64:", log2err)
+    for name, fit_f64 in (("2^f - 1 (tanh)", fit_expm1_f64), ("log", fit_log_f64)):
+        coefs, log2err = fit_f64()
+        for j, c in enumerate(coefs):
+            print(f"{name} coefficient {j}", float.hex(c))
+        print(f"log2 of the max weighted error of {name}:", log2err)
 
 
 if __name__ == "__main__":

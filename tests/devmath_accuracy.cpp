@@ -66,6 +66,17 @@ static long double gelu_exact(long double v)
     return v / (1.0L + std::exp(-2.0L * inner));
 }
 
+static double exp_z(float v) { return v >= -104.0f && v <= 89.0f ? mfh_exp_z(v) : NAN; }
+static double log_z(float v) { return v >= 0x1p-126f && v <= 0x1.fffffep127f ? mfh_log_z(v) : NAN; }
+// past 2^-12; below it the form gives v itself
+static double tanh_z(float v)
+{
+    return std::fabs(v) > 0x1p-12f ? std::copysign(mfh_tanh_z(std::fmin(std::fabs(v), 20.0f)), (double)v) : NAN;
+}
+static long double exp_exact(long double v) { return std::exp(v); }
+static long double log_exact(long double v) { return std::log(v); }
+static long double tanh_exact(long double v) { return std::tanh(v); }
+
 static uint32_t bits_of(float f)
 {
     uint32_t u;
@@ -84,6 +95,9 @@ int main(int argc, char** argv)
         {"sigmoid_p", 15, mfh_sigmoid_p, 1, mfh_sigmoid_cr, mfh_sigmoid_ref, sigmoid_z, sigmoid_exact},
         {"silu_p", 17, mfh_silu_p, 1, mfh_silu_cr, mfh_silu_ref, silu_z, silu_exact},
         {"gelu_p", 18, mfh_gelu_p, 1, mfh_gelu_cr, mfh_gelu_ref, gelu_z, gelu_exact},
+        {"exp_p", 12, mfh_exp_p, 1, mfh_exp_cr, mfh_exp_ref, exp_z, exp_exact},
+        {"log_p", 13, mfh_log_p, 1, mfh_log_cr, mfh_log_ref, log_z, log_exact},
+        {"tanh_p", 16, mfh_tanh_p, 1, mfh_tanh_cr, mfh_tanh_ref, tanh_z, tanh_exact},
     };
     const char* only = argc > 3 ? argv[3] : nullptr;
     for (const Fn& f : fns) {
