@@ -618,7 +618,10 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     // MFH_FUSION_PRECISE): two items per thread give a tanh chain 4%, an exp
     // and log chain 4% over f32 and 1% over bf16, a sigmoid chain 0-3% and the
     // precise SwiGLU chain 5.6% (the precise gelu chain -1%, within the noise
-    // of six alternating runs).  SwiGLU, Silu, add/mul chains and (since its 2^f runs on
+    // of six alternating runs).  f32 chains of two or more full operands have
+    // 32 bytes per lane in flight with one item and take one: silu(gate) * up
+    // over f32 [2048, 14336] 54.6 us against 56.7 with two, [512, 32000] 31.7
+    // against 33.2.  SwiGLU, Silu, add/mul chains and (since its 2^f runs on
     // v_exp_f32) the gelu chain over 16 bits lose 2-6% with two, and the
     // reference forms inline (MFH_FUSION_NO_ROUNDING_TEST) gain nothing.
     // Workgroups of one wave (kFusedThreads).  mfh_set_launch_config("fused",
@@ -637,7 +640,10 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
         if (is_fast_activation(node.type) ? rounded || (!precise && node.type == kNodeSigmoid)
                                           : is_transcendental(node.type) && (rounded || !precise))
             f64_fast = true;
-    const int unroll = items_per_thread(Kern::kFused) > 0 ? items_per_thread(Kern::kFused) : f64_fast ? 2 : 1;
+    int full_operands = 0;
+    for (int k = 0; k < n_inputs; k++) full_operands += inputs[k].mode == MFH_OPERAND_FULL;
+    const bool two_items = f64_fast && !(vec == 4 && full_operands >= 2);
+    const int unroll = items_per_thread(Kern::kFused) > 0 ? items_per_thread(Kern::kFused) : two_items ? 2 : 1;
     const int auto_bpc = kOneShotBlocksPerCu;
     const int block = threads_per_block(Kern::kFused) > 0 ? threads_per_block(Kern::kFused) : kFusedThreads;
     // Non-temporal loads for the streamed (full-length) operands when the
