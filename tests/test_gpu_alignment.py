@@ -105,3 +105,32 @@ def test_axpy_broadcast_linspace(dt, pads):
     same(got, O.encode(O.scalar_broadcast(O.decode(x, dt), 0.37, "mul"), dt), f"broadcast {dt} {pads}")
     got = run(lambda o, i: M.linspace(o, dt, N, -3.5, 11.0, True, stream()), x, N * SIZE[dt], pads)
     same(got, O.encode(O.linspace(-3.5, 11.0, N, True), dt), f"linspace {dt} {pads}")
+
+
+@pytest.mark.parametrize("pads", PADS[:4])
+@pytest.mark.parametrize("n", [1, 31, 4095, 4096, 4097, 3 * 4096 + 33])
+@pytest.mark.parametrize("out_dt", [O.F8E4M3, O.F8E5M2, O.INT8, O.INT4])
+def test_int4_sources_by_table(out_dt, n, pads):
+    # whole wave chunks of 4096 nibbles and the element tail; every byte value
+    packed = np.resize(np.random.default_rng(n).permutation(256).astype(np.uint8), (n + 1) // 2)
+    got = run(lambda o, i: M.convert(o, out_dt, i, O.INT4, n, stream()), packed,
+              (n + 1) // 2 if out_dt == O.INT4 else n, pads)
+    if out_dt == O.INT4:
+        want = O.bytes_to_i4(O.INT4, packed, n)
+    elif out_dt == O.INT8:
+        want = O.bytes_to_i8(O.INT4, packed)[:n]
+    else:
+        want = O.f32_to_fp8(O.bytes_to_f32(O.INT4, packed), out_dt)[:n]
+    same(got, want, f"i4->{out_dt} n={n} {pads}")
+
+
+@pytest.mark.parametrize("in_dt", [O.F8E4M3, O.F8E5M2])
+@pytest.mark.parametrize("out_dt", [O.F8E4M3, O.F8E5M2, O.INT8, O.INT4])
+def test_fp8_sources_every_code(in_dt, out_dt):
+    # every code, NaN and infinities among them, through whole chunks and the tail
+    n = 2 * 4096 + 77
+    a = np.resize(np.arange(256, dtype=np.uint8), n)
+    got = run(lambda o, i: M.convert(o, out_dt, i, in_dt, n, stream()), a, (n + 1) // 2 if out_dt == O.INT4 else n, (0, 0))
+    want = (O.bytes_to_i4(in_dt, a, n) if out_dt == O.INT4 else O.bytes_to_i8(in_dt, a) if out_dt == O.INT8
+            else O.f32_to_fp8(O.bytes_to_f32(in_dt, a), out_dt))
+    same(got, want, f"{in_dt}->{out_dt}")
