@@ -586,6 +586,48 @@ MFH_DEV mfh_u32 word_reg(const mfh_u32* w, int j)
     }
 }
 
+// How the encoders below split n elements over waves.  A wave takes chunks of
+// 256 pieces of P elements, lane l the pieces l, l + 64, l + 128 and l + 192;
+// the whole pieces after the last whole chunk go to waves of their own, one
+// piece per lane, and the fewer than P elements after those to the first
+// workgroup.  Left to an element loop of the chunks' waves, what follows the
+// last chunk of a small cast was one serial chain: MI355X, 8190 elements
+// e4m3 -> e5m2 2.1 us (15.5 so), Int4 -> e4m3 1.9 (11.1), int8 -> Int4 1.95
+// (7.7), bf16 -> e4m3 2.0 (3.8).  Below kSpread pieces, about what fills the
+// chip's wave slots with one piece per lane, there are no chunks: 2^19
+// elements e4m3 -> e5m2 2.1 us (2.9 in chunks), bf16 -> e4m3 2.08 (2.16).
+// Large casts are unchanged but for Int4 ones that stay within the Infinity
+// Cache, 0.1-0.2 us longer (int8 -> Int4, 2^24 elements: 6.1, 5.9 before).
+struct WaveSplit {
+    static constexpr int kChunk = 64 * 4;  // in pieces
+    static constexpr mfh_i64 kSpread = 1 << 17;
+    mfh_i64 chunks, units;  // units: chunks, then 64 pieces each
+    WaveSplit(mfh_i64 n, int elems)
+    {
+        const mfh_i64 pieces = n / elems;
+        chunks = pieces < kSpread ? 0 : pieces / kChunk;
+        units = chunks + (pieces - chunks * kChunk + 63) / 64;
+    }
+};
+
+// Runs step(first, U) for every unit of the calling wave, which takes the
+// pieces first + 64 q + lane, q < U (an integral constant); a piece past the
+// last one is left out.  Returns the number of pieces.  The chunk count comes
+// with the launch, so that a chunk's loads wait for no arithmetic on n: f32 ->
+// e4m3 of 2^24 elements 13.9 us, 14.0 with the count worked out per wave.
+template <int BS, int P, typename F>
+MFH_DEV mfh_i64 for_units(mfh_i64 n, mfh_i64 chunks, F&& step)
+{
+    const mfh_u32 lane = threadIdx.x & 63u;
+    const mfh_i64 waves = (mfh_i64)gridDim.x * (BS / 64);
+    mfh_i64 c = (mfh_i64)blockIdx.x * (BS / 64) + (threadIdx.x >> 6);
+    for (; c < chunks; c += waves) step(c * WaveSplit::kChunk, std::integral_constant<int, 4>{});
+    const mfh_i64 pieces = (mfh_i64)((mfh_u64)n / P);
+    for (mfh_i64 first = chunks * WaveSplit::kChunk + (c - chunks) * 64; first < pieces; first += waves * 64)
+        if (first + lane < pieces) step(first, std::integral_constant<int, 1>{});
+    return pieces;
+}
+
 // Int4 -> one byte per element.  The sixteen values' codes sit in four words
 // (codes of 0..7, then of -8..-1), and v_perm_b32 looks four of them up at a
 // time, so no element is decoded.
@@ -604,25 +646,21 @@ MFH_DEV mfh_u32 nibble_codes(mfh_u32 x)  // x: four nibbles, one per byte
     return (__builtin_amdgcn_perm(t[1], t[0], sel) & ~negative) | (__builtin_amdgcn_perm(t[3], t[2], sel) & negative);
 }
 
-// A wave takes chunks of 4096 elements, lane l the 8-byte pieces l, l + 64,
-// l + 128 and l + 192 of the chunk, each one 16-byte store.  MI355X, 2^26
+// Pieces of 8 bytes (WaveSplit), each one 16-byte store.  MI355X, 2^26
 // elements: Int4 -> e4m3 15.6 us, int8 15.4 (26.2 and 17.8 element by element);
 // FP8 sources of k_encode_byte_wave run e4m3 -> e5m2 in 25.4 us (58.8 so).
 template <int ENC, int BS>
 __global__ __launch_bounds__(BS) void k_encode_byte_int4(const mfh_u8* __restrict__ in, mfh_u8* __restrict__ out,
-                                                             mfh_i64 n)
+                                                             mfh_i64 n, mfh_i64 chunks)
 {
-    constexpr int kPieces = 4;
-    constexpr mfh_i64 kChunk = 64 * kPieces * 16;
-    const int lane = (int)threadIdx.x & 63;
-    const mfh_i64 waves = (mfh_i64)gridDim.x * (BS / 64);
-    const mfh_i64 nchunks = n / kChunk;
-    for (mfh_i64 c = (mfh_i64)blockIdx.x * (BS / 64) + (threadIdx.x >> 6); c < nchunks; c += waves) {
-        u32x2 x[kPieces];
+    const mfh_u32 lane = threadIdx.x & 63u;
+    const mfh_i64 pieces = for_units<BS, 16>(n, chunks, [&](mfh_i64 first, auto count) {
+        constexpr int U = decltype(count)::value;
+        u32x2 x[U];
 #pragma unroll
-        for (int q = 0; q < kPieces; q++) x[q] = load8<false>(in + c * (kChunk / 2) + (q * 64 + lane) * 8);
+        for (int q = 0; q < U; q++) x[q] = load8<false>(in + first * 8 + (q * 64 + lane) * 8);
 #pragma unroll
-        for (int q = 0; q < kPieces; q++) {
+        for (int q = 0; q < U; q++) {
             u32x4 o;
 #pragma unroll
             for (int h = 0; h < 2; h++) {
@@ -631,12 +669,11 @@ __global__ __launch_bounds__(BS) void k_encode_byte_int4(const mfh_u8* __restric
                 o[2 * h] = __builtin_amdgcn_perm(odd, even, 0x05010400u);
                 o[2 * h + 1] = __builtin_amdgcn_perm(odd, even, 0x07030602u);
             }
-            store16(out + c * kChunk + (q * 64 + lane) * 16, o);
+            store16(out + first * 16 + (q * 64 + lane) * 16, o);
         }
-    }
-    const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
-    for (mfh_i64 i = nchunks * kChunk + (mfh_i64)blockIdx.x * BS + threadIdx.x; i < n; i += stride)
-        out[i] = (mfh_u8)byte_at<kInt4, ENC>(in, i);
+    });
+    const mfh_i64 i = pieces * 16 + threadIdx.x;
+    if (blockIdx.x == 0 && i < n) out[i] = (mfh_u8)byte_at<kInt4, ENC>(in, i);
 }
 
 // Whether the encoders stream their source (non-temporal loads).  Where it
@@ -647,47 +684,40 @@ __global__ __launch_bounds__(BS) void k_encode_byte_int4(const mfh_u8* __restric
 bool streamed_source(const void* in) { return (reinterpret_cast<uintptr_t>(in) & 15u) == 0; }
 
 // Unpacked dtype -> one byte per element with every load instruction
-// of a wave reading 1 KiB contiguously: a wave takes chunks of 4 KiB of
-// source, lane l the 16-byte pieces l, l + 64, l + 128 and l + 192 of its
-// chunk, and writes the 16 / size output bytes of each piece next to its
-// neighbours' (16-, 8-, 4- or 2-byte stores).  Lanes taking two adjacent
+// of a wave reading 1 KiB contiguously: pieces of 16 source bytes (WaveSplit),
+// whose 16 / size output bytes go next to the neighbouring lanes' (16-, 8-,
+// 4- or 2-byte stores).  Lanes taking two adjacent
 // pieces each, so that 2-byte sources store 16 bytes at a time, split every
 // load instruction over 2 KiB: bf16 -> e4m3 ran 4% slower that way.  One lane
 // taking 16 consecutive elements (64 bytes of f32) spreads each load
-// instruction over 4 KiB: f32 -> e4m3 ran at 4.4 TB/s that way.  Elements
-// past the last whole chunk run the element loop.
+// instruction over 4 KiB: f32 -> e4m3 ran at 4.4 TB/s that way.
 template <int IN, int ENC, int BS, bool NT>
 __global__ __launch_bounds__(BS) void k_encode_byte_wave(const void* __restrict__ in, mfh_u8* __restrict__ out,
-                                                             mfh_i64 n)
+                                                             mfh_i64 n, mfh_i64 chunks)
 {
     constexpr int S = size_of<IN>();
-    constexpr int P = 16 / S;          // elements (and output bytes) per 16-byte piece
-    constexpr int kPieces = 4;         // pieces per lane per chunk
-    constexpr mfh_i64 kChunk = 64 * kPieces * P;  // elements per wave chunk
-    const int lane = (int)threadIdx.x & 63;
-    const mfh_i64 waves = (mfh_i64)gridDim.x * (BS / 64);
-    const mfh_i64 nchunks = n / kChunk;
-    for (mfh_i64 c = (mfh_i64)blockIdx.x * (BS / 64) + (threadIdx.x >> 6); c < nchunks; c += waves) {
-        u32x4 x[kPieces];
+    constexpr int P = 16 / S;  // elements (and output bytes) per 16-byte piece
+    const mfh_u32 lane = threadIdx.x & 63u;
+    const mfh_i64 pieces = for_units<BS, P>(n, chunks, [&](mfh_i64 first, auto count) {
+        constexpr int U = decltype(count)::value;
+        u32x4 x[U];
 #pragma unroll
-        for (int q = 0; q < kPieces; q++)
-            x[q] = load16<NT>(static_cast<const u32x4_any*>(in) + c * (64 * kPieces) + q * 64 + lane);
+        for (int q = 0; q < U; q++) x[q] = load16<NT>(static_cast<const u32x4_any*>(in) + first + (q * 64 + lane));
 #pragma unroll
-        for (int q = 0; q < kPieces; q++) {
+        for (int q = 0; q < U; q++) {
             const mfh_u32 w[4] = {x[q][0], x[q][1], x[q][2], x[q][3]};
             mfh_u32 code[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
             for (int j = 0; j < (P + 3) / 4; j++) code[j] = word_reg<IN, ENC, P>(w, j);
-            mfh_u8* o = out + c * kChunk + (mfh_i64)(q * 64 + lane) * P;
+            mfh_u8* o = out + first * P + (q * 64 + lane) * P;
             if constexpr (P == 16) store16(o, u32x4{code[0], code[1], code[2], code[3]});
             else if constexpr (P == 8) store8(o, u32x2{code[0], code[1]});
             else if constexpr (P == 4) store4(o, code[0]);
             else store2(o, code[0]);
         }
-    }
-    const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
-    for (mfh_i64 i = nchunks * kChunk + (mfh_i64)blockIdx.x * BS + threadIdx.x; i < n; i += stride)
-        out[i] = (mfh_u8)byte_at<IN, ENC>(in, i);
+    });
+    const mfh_i64 i = pieces * P + threadIdx.x;
+    if (blockIdx.x == 0 && i < n) out[i] = (mfh_u8)byte_at<IN, ENC>(in, i);
 }
 
 // Workgroup size of a cast unless the launch config sets one.  Measured at
@@ -707,13 +737,13 @@ template <int ENC, int BS>
 int launch_encode_byte_wave(const Device* dev, mfh_u8* out, const void* in, int in_dt, int64_t n, int size,
                             hipStream_t stream)
 {
-    const int64_t chunk_elems = 64 * 4 * (16 / size);
-    const unsigned grid = grid_for(std::max<int64_t>(n / chunk_elems, 1) * 64, dev, Kern::kConvert, 1, BS);
+    const WaveSplit split(n, 16 / size);
+    const unsigned grid = grid_for(split.units * 64, dev, Kern::kConvert, 1, BS);
     switch (in_dt) {
 #define MFH_ENCODE_WAVE_CASE(DT) \
     case DT: \
-        if (streamed_source(in)) k_encode_byte_wave<DT, ENC, BS, true><<<grid, BS, 0, stream>>>(in, out, n); \
-        else k_encode_byte_wave<DT, ENC, BS, false><<<grid, BS, 0, stream>>>(in, out, n); \
+        if (streamed_source(in)) k_encode_byte_wave<DT, ENC, BS, true><<<grid, BS, 0, stream>>>(in, out, n, split.chunks); \
+        else k_encode_byte_wave<DT, ENC, BS, false><<<grid, BS, 0, stream>>>(in, out, n, split.chunks); \
         break;
         MFH_ENCODE_WAVE_CASE(kFloat64)
         MFH_ENCODE_WAVE_CASE(kFloat32)
@@ -748,8 +778,9 @@ int launch_encode_byte(const Device* dev, mfh_u8* out, const void* in, int in_dt
         return fail(MFH_ERR_DTYPE_UNSUPPORTED, "mfh_convert: input dtype %s is not supported", dtype_name(in_dt));
     return with_block(cast_threads(in_dt, 1), [&](auto block) {
         constexpr int BS = decltype(block)::value;
-        const unsigned grid = grid_for(std::max<int64_t>(n / 4096, 1) * 64, dev, Kern::kConvert, 1, BS);
-        k_encode_byte_int4<ENC, BS><<<grid, BS, 0, stream>>>(static_cast<const mfh_u8*>(in), out, n);
+        const WaveSplit split(n, 16);
+        const unsigned grid = grid_for(split.units * 64, dev, Kern::kConvert, 1, BS);
+        k_encode_byte_int4<ENC, BS><<<grid, BS, 0, stream>>>(static_cast<const mfh_u8*>(in), out, n, split.chunks);
         return launch_status("k_encode_byte_int4");
     });
 }
@@ -812,43 +843,35 @@ __global__ __launch_bounds__(kBlock) void k_copy_int4(const mfh_u8* __restrict__
         out[b] = b < whole ? in[b] : in[b] & 0x0f;
 }
 
-// Unpacked sources, laid out as k_encode_byte_wave: a wave takes 4 KiB
-// of source, lane l its 16-byte pieces l, l + 64, l + 128 and l + 192, so
-// every load instruction reads 1 KiB contiguously; the 16 / size elements of
+// Unpacked sources, laid out as k_encode_byte_wave: the 16 / size elements of
 // a piece leave as 8 / size bytes of nibbles next to the neighbours' ones.
-// Elements past the last whole chunk run the byte loop.
 template <int IN, int BS, bool NT>
 __global__ __launch_bounds__(BS) void k_encode_int4_wave(const void* __restrict__ in, mfh_u8* __restrict__ out,
-                                                             mfh_i64 n)
+                                                             mfh_i64 n, mfh_i64 chunks)
 {
     constexpr int S = size_of<IN>();
     constexpr int P = 16 / S;  // elements per 16-byte piece
-    constexpr int kPieces = 4;
-    constexpr mfh_i64 kChunk = 64 * kPieces * P;
-    const int lane = (int)threadIdx.x & 63;
-    const mfh_i64 waves = (mfh_i64)gridDim.x * (BS / 64);
-    const mfh_i64 nchunks = n / kChunk;
-    for (mfh_i64 c = (mfh_i64)blockIdx.x * (BS / 64) + (threadIdx.x >> 6); c < nchunks; c += waves) {
-        u32x4 x[kPieces];
+    const mfh_u32 lane = threadIdx.x & 63u;
+    const mfh_i64 pieces = for_units<BS, P>(n, chunks, [&](mfh_i64 first, auto count) {
+        constexpr int U = decltype(count)::value;
+        u32x4 x[U];
 #pragma unroll
-        for (int q = 0; q < kPieces; q++)
-            x[q] = load16<NT>(static_cast<const u32x4_any*>(in) + c * (64 * kPieces) + q * 64 + lane);
+        for (int q = 0; q < U; q++) x[q] = load16<NT>(static_cast<const u32x4_any*>(in) + first + (q * 64 + lane));
 #pragma unroll
-        for (int q = 0; q < kPieces; q++) {
+        for (int q = 0; q < U; q++) {
             const mfh_u32 w[4] = {x[q][0], x[q][1], x[q][2], x[q][3]};
             mfh_u32 code[2] = {0u, 0u};
 #pragma unroll
             for (int k = 0; k < P; k++) code[k >> 3] |= nibble_reg<IN>(w, k) << (4 * (k & 7));
-            mfh_u8* o = out + (c * kChunk + (mfh_i64)(q * 64 + lane) * P) / 2;
+            mfh_u8* o = out + first * P / 2 + (q * 64 + lane) * P / 2;
             if constexpr (P == 16) store8(o, u32x2{code[0], code[1]});
             else if constexpr (P == 8) store4(o, code[0]);
             else if constexpr (P == 4) store2(o, code[0]);
             else *o = (mfh_u8)code[0];
         }
-    }
-    const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
-    const mfh_i64 nbytes = (n + 1) / 2;
-    for (mfh_i64 b = nchunks * kChunk / 2 + (mfh_i64)blockIdx.x * BS + threadIdx.x; b < nbytes; b += stride) {
+    });
+    const mfh_i64 b = pieces * P / 2 + threadIdx.x;
+    if (blockIdx.x == 0 && b < (n + 1) / 2) {
         const mfh_u32 lo = nibble_at<IN>(in, 2 * b);
         const mfh_u32 hi = 2 * b + 1 < n ? nibble_at<IN>(in, 2 * b + 1) : 0u;
         out[b] = (mfh_u8)(lo | (hi << 4));
@@ -859,13 +882,13 @@ template <int BS>
 int launch_encode_int4_wave(const Device* dev, mfh_u8* out, const void* in, int in_dt, int64_t n, int size,
                             hipStream_t stream)
 {
-    const int64_t chunk_elems = 64 * 4 * (16 / size);
-    const unsigned grid = grid_for(std::max<int64_t>(n / chunk_elems, 1) * 64, dev, Kern::kConvert, 1, BS);
+    const WaveSplit split(n, 16 / size);
+    const unsigned grid = grid_for(split.units * 64, dev, Kern::kConvert, 1, BS);
     switch (in_dt) {
 #define MFH_ENCODE_I4_WAVE_CASE(DT) \
     case DT: \
-        if (streamed_source(in)) k_encode_int4_wave<DT, BS, true><<<grid, BS, 0, stream>>>(in, out, n); \
-        else k_encode_int4_wave<DT, BS, false><<<grid, BS, 0, stream>>>(in, out, n); \
+        if (streamed_source(in)) k_encode_int4_wave<DT, BS, true><<<grid, BS, 0, stream>>>(in, out, n, split.chunks); \
+        else k_encode_int4_wave<DT, BS, false><<<grid, BS, 0, stream>>>(in, out, n, split.chunks); \
         break;
         MFH_ENCODE_I4_WAVE_CASE(kFloat64)
         MFH_ENCODE_I4_WAVE_CASE(kFloat32)

@@ -111,7 +111,7 @@ def test_axpy_broadcast_linspace(dt, pads):
 @pytest.mark.parametrize("n", [1, 31, 4095, 4096, 4097, 3 * 4096 + 33])
 @pytest.mark.parametrize("out_dt", [O.F8E4M3, O.F8E5M2, O.INT8, O.INT4])
 def test_int4_sources_by_table(out_dt, n, pads):
-    # whole wave chunks of 4096 nibbles and the element tail; every byte value
+    # whole 16-nibble pieces and the element tail; every byte value
     packed = np.resize(np.random.default_rng(n).permutation(256).astype(np.uint8), (n + 1) // 2)
     got = run(lambda o, i: M.convert(o, out_dt, i, O.INT4, n, stream()), packed,
               (n + 1) // 2 if out_dt == O.INT4 else n, pads)
@@ -127,10 +127,33 @@ def test_int4_sources_by_table(out_dt, n, pads):
 @pytest.mark.parametrize("in_dt", [O.F8E4M3, O.F8E5M2])
 @pytest.mark.parametrize("out_dt", [O.F8E4M3, O.F8E5M2, O.INT8, O.INT4])
 def test_fp8_sources_every_code(in_dt, out_dt):
-    # every code, NaN and infinities among them, through whole chunks and the tail
+    # every code, NaN and infinities among them, through whole pieces and the tail
     n = 2 * 4096 + 77
     a = np.resize(np.arange(256, dtype=np.uint8), n)
     got = run(lambda o, i: M.convert(o, out_dt, i, in_dt, n, stream()), a, (n + 1) // 2 if out_dt == O.INT4 else n, (0, 0))
     want = (O.bytes_to_i4(in_dt, a, n) if out_dt == O.INT4 else O.bytes_to_i8(in_dt, a) if out_dt == O.INT8
             else O.f32_to_fp8(O.bytes_to_f32(in_dt, a), out_dt))
     same(got, want, f"{in_dt}->{out_dt}")
+
+
+@pytest.mark.parametrize("pads", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("out_dt", [O.F8E4M3, O.INT8, O.INT4])
+@pytest.mark.parametrize("in_dt", [O.FLOAT64, O.FLOAT32, O.BFLOAT16, O.INT8, O.F8E5M2, O.INT4])
+def test_encode_wave_split(in_dt, out_dt, pads):
+    # 64 pieces per wave, from 2^17 pieces on whole chunks of 256 first, then fewer elements than a piece
+    piece = 16 // SIZE.get(in_dt, 1)
+    counts = [pieces * piece + d for pieces in (0, 1, 63, 64, 65, 256, 257) for d in (-1, 0, 1, piece // 2)]
+    counts += [(1 << 17) * piece - 1, (1 << 17) * piece, ((1 << 17) + 256 + 65) * piece + 1]
+    for n in sorted({n for n in counts if n > 0}):
+        rng = np.random.default_rng(n)
+        if in_dt == O.INT4:
+            a = rng.integers(0, 256, (n + 1) // 2, dtype=np.uint8)
+        elif in_dt == O.INT8:
+            a = rng.integers(-128, 128, n).astype(np.int8)
+        else:
+            a = rng.integers(0, 256, n, dtype=np.uint8) if in_dt == O.F8E5M2 else rng.normal(0, 40, n)
+            a = O.encode(a.astype(np.float32), in_dt) if in_dt in (O.FLOAT32, O.BFLOAT16) else a
+        got = run(lambda o, i: M.convert(o, out_dt, i, in_dt, n, stream()), a, (n + 1) // 2 if out_dt == O.INT4 else n, pads)
+        want = (O.bytes_to_i4(in_dt, a, n) if out_dt == O.INT4 else O.bytes_to_i8(in_dt, a)[:n] if out_dt == O.INT8
+                else O.f32_to_fp8(O.bytes_to_f32(in_dt, a), out_dt)[:n])
+        same(got, want, f"{in_dt}->{out_dt} n={n} {pads}")
