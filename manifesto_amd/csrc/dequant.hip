@@ -75,7 +75,7 @@ MFH_DEV mfh_u32 fp8_bits_hw(mfh_u32 code, bool e5m2)
     return f != f ? nan : mfh_bits(f);
 }
 
-template <int OUT, int U, int BS>
+template <int OUT, int U, int BS, bool DWORDS>
 __global__ __launch_bounds__(BS) void k_dequant_fp8(const mfh_u8* __restrict__ in,
                                                         void* __restrict__ out, mfh_i64 n,
                                                         float scale, int fmt)
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(BS) void k_dequant_fp8(const mfh_u8* __restrict__ i
     for (; c < nchunks; c += gridDim.x) {
         if (c != (mfh_i64)blockIdx.x) load(c);
         const mfh_i64 first = c * kChunk;
-        const StreamOut dst(static_cast<char*>(out) + first * 16, nitems - first);
+        const StreamOut<DWORDS> dst(static_cast<char*>(out) + first * 16, nitems - first);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int j = u * BS + (int)t;
@@ -242,7 +242,7 @@ struct Int4Scales {
 // stores, a 64-bit division per element), which every group that is not a
 // power of two took; with groups of 128 the shift runs 21.5 us where the
 // multiplication ran 21.6-21.9.
-template <int OUT, int SDT, int U, int BS, bool ANY>
+template <int OUT, int SDT, int U, int BS, bool ANY, bool DWORDS>
 MFH_DEV void dequant_int4(const mfh_u8* __restrict__ packed, const void* __restrict__ scales,
                           void* __restrict__ out, mfh_i64 n, const Int4Group& group, bool vec_ok)
 {
@@ -284,7 +284,7 @@ MFH_DEV void dequant_int4(const mfh_u8* __restrict__ packed, const void* __restr
             s1[u] = ANY ? scale_value<SDT>(sb1[u]) : s[u];
         }
         // The buffer descriptor ends at the last item: stores past it are dropped.
-        const StreamOut dst(static_cast<char*>(out) + first * 16, nitems - first);
+        const StreamOut<DWORDS> dst(static_cast<char*>(out) + first * 16, nitems - first);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int j = u * BS + t;
@@ -316,22 +316,22 @@ MFH_DEV void dequant_int4(const mfh_u8* __restrict__ packed, const void* __restr
 // The two kernels take just the arguments they use: gfx950 preloads the first
 // 14 dwords into SGPRs, and the grid size that follows a longer list costs
 // every wave a scalar load ahead of its first vector load (0.5% at 147 MB).
-template <int OUT, int SDT, int U, int BS>
+template <int OUT, int SDT, int U, int BS, bool DWORDS>
 __global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ packed,
                                                          const void* __restrict__ scales,
                                                          void* __restrict__ out, mfh_i64 n, mfh_i64 size,
                                                          int shift, int vec_ok)
 {
-    dequant_int4<OUT, SDT, U, BS, false>(packed, scales, out, n, Int4Group{size, shift, 0u, 0u, 0.0}, vec_ok != 0);
+    dequant_int4<OUT, SDT, U, BS, false, DWORDS>(packed, scales, out, n, Int4Group{size, shift, 0u, 0u, 0.0}, vec_ok != 0);
 }
 
-template <int OUT, int SDT, int U, int BS>
+template <int OUT, int SDT, int U, int BS, bool DWORDS>
 __global__ __launch_bounds__(BS) void k_dequant_int4_any(const mfh_u8* __restrict__ packed,
                                                              const void* __restrict__ scales,
                                                              void* __restrict__ out, mfh_i64 n, mfh_u32 step,
                                                              mfh_u32 mul, double inverse, mfh_i64 size)
 {
-    dequant_int4<OUT, SDT, U, BS, true>(packed, scales, out, n, Int4Group{size, -1, step, mul, inverse}, true);
+    dequant_int4<OUT, SDT, U, BS, true, DWORDS>(packed, scales, out, n, Int4Group{size, -1, step, mul, inverse}, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -1061,6 +1061,8 @@ int by_out(int out_dt, A... args)
     }
 }
 
+bool dword_aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 3u) == 0; }
+
 template <int OUT>
 struct Fp8Launch {
     static int run(const Device* dev, void* out, const void* in, int fmt, int64_t n, float scale,
@@ -1069,13 +1071,18 @@ struct Fp8Launch {
         constexpr int codes = OUT == kFloat32 ? 4 : 8;
         const int64_t items = std::max<int64_t>(n / codes, 1);
         const mfh_u8* src = static_cast<const mfh_u8*>(in);
+        if (!dword_aligned(out)) {  // in the default shape only
+            k_dequant_fp8<OUT, 2, 128, false>
+                <<<grid_for(items, dev, Kern::kFp8, 2, 128), 128, 0, stream>>>(src, out, n, scale, fmt);
+            return launch_status("k_dequant_fp8");
+        }
         const int u = items_per_thread(Kern::kFp8);
         return with_block(threads_per_block(Kern::kFp8), [&](auto block) {
             constexpr int BS = decltype(block)::value;
             const unsigned grid = grid_for(items, dev, Kern::kFp8, u, BS);
-            if (u == 4) k_dequant_fp8<OUT, 4, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
-            else if (u == 2) k_dequant_fp8<OUT, 2, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
-            else k_dequant_fp8<OUT, 1, BS><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
+            if (u == 4) k_dequant_fp8<OUT, 4, BS, true><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
+            else if (u == 2) k_dequant_fp8<OUT, 2, BS, true><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
+            else k_dequant_fp8<OUT, 1, BS, true><<<grid, BS, 0, stream>>>(src, out, n, scale, fmt);
             return launch_status("k_dequant_fp8");
         });
     }
@@ -1098,19 +1105,24 @@ struct Int4Launch {
         const int vec_ok = size >= elems;
         const bool any = vec_ok && group.shift < 0;
         const int64_t items = vec_ok ? std::max<int64_t>(n / elems, 1) : n;
-        const int u = items_per_thread(Kern::kInt4);
         const mfh_u8* p = static_cast<const mfh_u8*>(packed);
+        if (!dword_aligned(out)) {  // in the default shape only
+            launch<2, 512, false>(grid_for(items, dev, Kern::kInt4, 2, 512), p, scales, scale_dt, out, n, group, vec_ok,
+                                  any, stream);
+            return launch_status("k_dequant_int4");
+        }
+        const int u = items_per_thread(Kern::kInt4);
         return with_block_to_512(threads_per_block(Kern::kInt4), [&](auto block) {
             constexpr int BS = decltype(block)::value;
             const unsigned grid = grid_for(items, dev, Kern::kInt4, u, BS);
-            if (u == 4) launch<4, BS>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
-            else if (u == 2) launch<2, BS>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
-            else launch<1, BS>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
+            if (u == 4) launch<4, BS, true>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
+            else if (u == 2) launch<2, BS, true>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
+            else launch<1, BS, true>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
             return launch_status("k_dequant_int4");
         });
     }
 
-    template <int U, int BS>
+    template <int U, int BS, bool DWORDS>
     static void launch(unsigned grid, const mfh_u8* p, const void* scales, int scale_dt, void* out, int64_t n,
                        const Int4Group& group, int vec_ok, bool any, hipStream_t stream)
     {
@@ -1118,10 +1130,10 @@ struct Int4Launch {
 #define MFH_INT4_CASE(DT)                                                                                           \
     case DT:                                                                                                        \
         if (any)                                                                                                    \
-            k_dequant_int4_any<OUT, DT, U, BS>                                                                      \
+            k_dequant_int4_any<OUT, DT, U, BS, DWORDS>                                                              \
                 <<<grid, BS, 0, stream>>>(p, scales, out, n, group.step, group.mul, group.inverse, group.size);     \
         else                                                                                                        \
-            k_dequant_int4<OUT, DT, U, BS>                                                                          \
+            k_dequant_int4<OUT, DT, U, BS, DWORDS>                                                                  \
                 <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift, vec_ok);                      \
         break;
             MFH_INT4_CASE(kFloat32)
@@ -1129,7 +1141,7 @@ struct Int4Launch {
             MFH_INT4_CASE(kBFloat16)
 #undef MFH_INT4_CASE
         default:
-            k_dequant_int4<OUT, kInvalid, U, BS>
+            k_dequant_int4<OUT, kInvalid, U, BS, DWORDS>
                 <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift, vec_ok);
             break;
         }

@@ -107,21 +107,25 @@ __device__ inline void store2(void* p, mfh_u32 v) { __builtin_nontemporal_store(
 // against 5.8 and 5.5 with plain stores; nt alone is 1-2% slower, sc1 alone
 // 4-6%.  The descriptor's record count is the chunk's remaining bytes, so the
 // hardware drops anything past the end of the output.  A base that is not
-// dword-aligned takes global stores (nt), which any address allows.
+// dword-aligned (DWORDS = false) takes global stores (nt), which any address
+// allows.  The kernel is compiled for one of the two: choosing per store put
+// branches and both stores' code into every item, 0.1-0.2 us of each call whose
+// few workgroups wait for instruction fetches (Int4, groups of 128 -> bf16 on
+// MI355X: 2^16 elements 2.26 us, 2.46 so; 2^22 elements 3.09, 3.29 so).
+template <bool DWORDS>
 struct StreamOut {
     char* at;
     int64_t left;
-    bool dwords;
     __amdgpu_buffer_rsrc_t rsrc;
     __device__ StreamOut(char* base, int64_t items_left)
-        : at(base), left(items_left), dwords((reinterpret_cast<uintptr_t>(base) & 3u) == 0),
+        : at(base), left(items_left),
           rsrc(__builtin_amdgcn_make_buffer_rsrc(
               base, 0, (int)std::min<int64_t>(items_left * 16, 0x7fffffff), kBufferConfig))
     {
     }
     __device__ void store(int item, u32x4 v) const
     {
-        if (dwords) __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, item * 16, 0, kCachePolicy);
+        if constexpr (DWORDS) __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, item * 16, 0, kCachePolicy);
         else if (item < left) store16(at + (int64_t)item * 16, v);
     }
     // Word 3 of a raw (untyped) gfx9 buffer descriptor.

@@ -36,15 +36,17 @@ def test_split_items_with_scales_that_are_not_finite(group):
         int4_case(n, group, O.FLOAT32, out_dt, scales, rng)
 
 
+# pad 1 puts a 16-bit output off its dwords, which runs the default shape
+@pytest.mark.parametrize("pad", [0, 1])
 @pytest.mark.parametrize("items, threads", [(1, 64), (2, 128), (4, 512)])
-def test_launch_shapes(items, threads):
+def test_launch_shapes(items, threads, pad):
     rng = np.random.default_rng(items)
     try:
         M.set_launch_config("int4", 0, items)
         M.set_launch_threads("int4", threads)
-        for group in (100, 40001):
+        for group in (64, 100, 40001):
             n = 5 * 16384 + 7
-            int4_case(n, group, O.FLOAT16, O.BFLOAT16, rng.uniform(0.005, 0.02, n // group + 2).astype(np.float32), rng)
+            int4_case(n, group, O.FLOAT16, O.BFLOAT16, rng.uniform(0.005, 0.02, n // group + 2).astype(np.float32), rng, pad)
     finally:
         M.set_launch_config("int4", -1, -1)
         M.set_launch_threads("int4", -1)
