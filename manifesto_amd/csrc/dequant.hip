@@ -229,9 +229,33 @@ struct Int4Scales {
     }
 };
 
+// Elements `first` to n one by one.
+template <int OUT, int SDT, int BS>
+MFH_DEV void int4_elements(const mfh_u8* __restrict__ packed, const void* __restrict__ scales,
+                           void* __restrict__ out, mfh_i64 first, mfh_i64 n, mfh_i64 size)
+{
+    const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
+    for (mfh_i64 i = first + (mfh_i64)blockIdx.x * BS + threadIdx.x; i < n; i += stride) {
+        mfh_u32 byte = packed[i >> 1];
+        float q = (float)mfh_int4_at(byte, (mfh_u32)(i & 1));
+        float s = load_scale<SDT>(scales, i / size);
+        store_one<OUT>(out, i, encode_one<OUT>(mfh_scale_mul(q, s)));
+    }
+}
+
+// Groups smaller than an item, element by element.  A kernel of its own: beside
+// the item loop below, bf16 of 2^24 elements in groups of 3 took 28.4 us, 25.7
+// so.
+template <int OUT, int SDT, int BS>
+__global__ __launch_bounds__(BS) void k_dequant_int4_small(const mfh_u8* __restrict__ packed,
+                                                               const void* __restrict__ scales,
+                                                               void* __restrict__ out, mfh_i64 n, mfh_i64 size)
+{
+    int4_elements<OUT, SDT, BS>(packed, scales, out, 0, n, size);
+}
+
 // Item = 8 nibbles (4 packed bytes, 16-bit output) or 4 nibbles (2 bytes, f32
-// output) -> one 16-byte store.  Groups smaller than an item run the element
-// loop.  A block of BS threads takes chunks of BS * U consecutive items
+// output) -> one 16-byte store, for groups of at least an item.  A block of BS threads takes chunks of BS * U consecutive items
 // (thread t holds items t, t + BS, ...), one-shot by default, with streaming
 // stores (StreamOut) addressed from the chunk's first item.  The chunks are
 // contiguous, as FP8's: a grid-stride loop whose U items per thread sat a
@@ -244,12 +268,12 @@ struct Int4Scales {
 // multiplication ran 21.6-21.9.
 template <int OUT, int SDT, int U, int BS, bool ANY, bool DWORDS>
 MFH_DEV void dequant_int4(const mfh_u8* __restrict__ packed, const void* __restrict__ scales,
-                          void* __restrict__ out, mfh_i64 n, const Int4Group& group, bool vec_ok)
+                          void* __restrict__ out, mfh_i64 n, const Int4Group& group)
 {
     constexpr int kElems = OUT == kFloat32 ? 4 : 8;
     constexpr mfh_i64 kChunk = (mfh_i64)BS * U;
     static_assert(kChunk * kElems <= (1 << 14), "a chunk spans at most 2^14 elements");
-    const mfh_i64 nitems = vec_ok ? n / kElems : 0;
+    const mfh_i64 nitems = n / kElems;
     const mfh_i64 nchunks = (nitems + kChunk - 1) / kChunk;
     const int t = (int)threadIdx.x;
     for (mfh_i64 c = blockIdx.x; c < nchunks; c += gridDim.x) {
@@ -304,13 +328,7 @@ MFH_DEV void dequant_int4(const mfh_u8* __restrict__ packed, const void* __restr
                                    encode_pair<OUT>(f[4], f[5]), encode_pair<OUT>(f[6], f[7])});
         }
     }
-    const mfh_i64 stride = (mfh_i64)gridDim.x * BS;
-    for (mfh_i64 i = nitems * kElems + (mfh_i64)blockIdx.x * BS + threadIdx.x; i < n; i += stride) {
-        mfh_u32 byte = packed[i >> 1];
-        float q = (float)mfh_int4_at(byte, (mfh_u32)(i & 1));
-        float s = load_scale<SDT>(scales, i / group.size);
-        store_one<OUT>(out, i, encode_one<OUT>(mfh_scale_mul(q, s)));
-    }
+    int4_elements<OUT, SDT, BS>(packed, scales, out, nitems * kElems, n, group.size);
 }
 
 // The two kernels take just the arguments they use: gfx950 preloads the first
@@ -320,9 +338,9 @@ template <int OUT, int SDT, int U, int BS, bool DWORDS>
 __global__ __launch_bounds__(BS) void k_dequant_int4(const mfh_u8* __restrict__ packed,
                                                          const void* __restrict__ scales,
                                                          void* __restrict__ out, mfh_i64 n, mfh_i64 size,
-                                                         int shift, int vec_ok)
+                                                         int shift)
 {
-    dequant_int4<OUT, SDT, U, BS, false, DWORDS>(packed, scales, out, n, Int4Group{size, shift, 0u, 0u, 0.0}, vec_ok != 0);
+    dequant_int4<OUT, SDT, U, BS, false, DWORDS>(packed, scales, out, n, Int4Group{size, shift, 0u, 0u, 0.0});
 }
 
 template <int OUT, int SDT, int U, int BS, bool DWORDS>
@@ -331,7 +349,7 @@ __global__ __launch_bounds__(BS) void k_dequant_int4_any(const mfh_u8* __restric
                                                              void* __restrict__ out, mfh_i64 n, mfh_u32 step,
                                                              mfh_u32 mul, double inverse, mfh_i64 size)
 {
-    dequant_int4<OUT, SDT, U, BS, true, DWORDS>(packed, scales, out, n, Int4Group{size, -1, step, mul, inverse}, true);
+    dequant_int4<OUT, SDT, U, BS, true, DWORDS>(packed, scales, out, n, Int4Group{size, -1, step, mul, inverse});
 }
 
 // ---------------------------------------------------------------------------
@@ -1102,29 +1120,41 @@ struct Int4Launch {
         // (step 1, an element-loop group, has no 32-bit multiplier and needs none)
         const uint64_t range = uint64_t(1) << 32;
         group.mul = (mfh_u32)(range / group.step + (range % group.step != 0));
-        const int vec_ok = size >= elems;
-        const bool any = vec_ok && group.shift < 0;
-        const int64_t items = vec_ok ? std::max<int64_t>(n / elems, 1) : n;
+        const bool small = size < elems;
+        const bool any = !small && group.shift < 0;
+        const int64_t items = small ? n : std::max<int64_t>(n / elems, 1);
         const mfh_u8* p = static_cast<const mfh_u8*>(packed);
-        if (!dword_aligned(out)) {  // in the default shape only
-            launch<2, 512, false>(grid_for(items, dev, Kern::kInt4, 2, 512), p, scales, scale_dt, out, n, group, vec_ok,
-                                  any, stream);
+        if (!small && !dword_aligned(out)) {  // in the default shape only
+            launch<2, 512, false>(grid_for(items, dev, Kern::kInt4, 2, 512), p, scales, scale_dt, out, n, group, any,
+                                  stream);
             return launch_status("k_dequant_int4");
         }
         const int u = items_per_thread(Kern::kInt4);
         return with_block_to_512(threads_per_block(Kern::kInt4), [&](auto block) {
             constexpr int BS = decltype(block)::value;
             const unsigned grid = grid_for(items, dev, Kern::kInt4, u, BS);
-            if (u == 4) launch<4, BS, true>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
-            else if (u == 2) launch<2, BS, true>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
-            else launch<1, BS, true>(grid, p, scales, scale_dt, out, n, group, vec_ok, any, stream);
+            if (small) launch_small<BS>(grid, p, scales, scale_dt, out, n, size, stream);
+            else if (u == 4) launch<4, BS, true>(grid, p, scales, scale_dt, out, n, group, any, stream);
+            else if (u == 2) launch<2, BS, true>(grid, p, scales, scale_dt, out, n, group, any, stream);
+            else launch<1, BS, true>(grid, p, scales, scale_dt, out, n, group, any, stream);
             return launch_status("k_dequant_int4");
         });
     }
 
+    template <int BS>
+    static void launch_small(unsigned grid, const mfh_u8* p, const void* scales, int scale_dt, void* out, int64_t n,
+                             int64_t size, hipStream_t stream)
+    {
+        switch (scale_dt) {
+        case kFloat32: k_dequant_int4_small<OUT, kFloat32, BS><<<grid, BS, 0, stream>>>(p, scales, out, n, size); break;
+        case kFloat16: k_dequant_int4_small<OUT, kFloat16, BS><<<grid, BS, 0, stream>>>(p, scales, out, n, size); break;
+        default: k_dequant_int4_small<OUT, kBFloat16, BS><<<grid, BS, 0, stream>>>(p, scales, out, n, size); break;
+        }
+    }
+
     template <int U, int BS, bool DWORDS>
     static void launch(unsigned grid, const mfh_u8* p, const void* scales, int scale_dt, void* out, int64_t n,
-                       const Int4Group& group, int vec_ok, bool any, hipStream_t stream)
+                       const Int4Group& group, bool any, hipStream_t stream)
     {
         switch (scale_dt) {
 #define MFH_INT4_CASE(DT)                                                                                           \
@@ -1134,15 +1164,15 @@ struct Int4Launch {
                 <<<grid, BS, 0, stream>>>(p, scales, out, n, group.step, group.mul, group.inverse, group.size);     \
         else                                                                                                        \
             k_dequant_int4<OUT, DT, U, BS, DWORDS>                                                                  \
-                <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift, vec_ok);                      \
+                <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift);                              \
         break;
             MFH_INT4_CASE(kFloat32)
             MFH_INT4_CASE(kFloat16)
             MFH_INT4_CASE(kBFloat16)
 #undef MFH_INT4_CASE
-        default:
+        default:  // mfh_convert: no scale, one group
             k_dequant_int4<OUT, kInvalid, U, BS, DWORDS>
-                <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift, vec_ok);
+                <<<grid, BS, 0, stream>>>(p, scales, out, n, group.size, group.shift);
             break;
         }
     }
