@@ -179,18 +179,24 @@ struct Int4Group {
 //
 // ANY = true, any other size of at least an item's elements: an item can hold
 // the end of one group and the start of the next, and reads both scales.  The
-// quotient for e0 by the rounded inverse is at most one off.  For groups up
-// to 2^15, x stays below 2^16, where the multiplication by 2^32 / step
-// rounded up divides exactly; a larger group takes steps of 2^16 and r' =
-// 2^16 - (elements to the group's end), as above.
-template <int ELEMS, bool ANY>
+// quotient for e0 by the rounded inverse is at most one off (the launcher sees
+// to it that it fits 32 bits).  For groups up to 2^15, x stays below 2^16,
+// where the multiplication by 2^32 / step rounded up divides exactly; a larger
+// group takes steps of 2^16 and r' = 2^16 - (elements to the group's end), as
+// above.  Every workgroup's scale loads wait for this division, so it stays
+// short: with 64-bit conversions and products for every group size a call of
+// 2^16 elements took 2.46 us (groups of 14336) and 2.66 (100000), 2.44 and 2.46
+// so.
+template <int ELEMS, mfh_i64 CHUNK, bool ANY>
 struct Int4Scales {
     mfh_i64 g0;
     mfh_u32 x0, step, mul;
     int shift;
 
-    __device__ Int4Scales(const Int4Group& group, mfh_i64 e0)
+    // of chunk c, whose first element is e0 = c * CHUNK
+    __device__ Int4Scales(const Int4Group& group, mfh_i64 c)
     {
+        const mfh_i64 e0 = c * CHUNK;
         if constexpr (!ANY) {
             g0 = e0 >> group.shift;
             const mfh_u64 r = (mfh_u64)(e0 - (g0 << group.shift));
@@ -199,17 +205,22 @@ struct Int4Scales {
             x0 = small_group ? (mfh_u32)r : to_next >= (1u << 20) ? 0u : (1u << 20) - (mfh_u32)to_next;
             shift = small_group ? group.shift : 20;
         } else {
-            const mfh_u64 q = (mfh_u64)((double)e0 * group.inverse);
-            g0 = (mfh_i64)((mfh_u64)__builtin_amdgcn_readfirstlane((mfh_u32)(q >> 32)) << 32 |
-                           (mfh_u32)__builtin_amdgcn_readfirstlane((mfh_u32)q));
-            mfh_i64 r = e0 - g0 * group.size;
-            if (r < 0) g0--, r += group.size;
-            if (r >= group.size) g0++, r -= group.size;
-            const mfh_i64 to_next = group.size - r;
             step = group.step;
             mul = group.mul;
-            x0 = step != Int4Group::kWide ? (mfh_u32)r
-                 : to_next >= (mfh_i64)Int4Group::kWide ? 0u : Int4Group::kWide - (mfh_u32)to_next;
+            const mfh_u32 q = __builtin_amdgcn_readfirstlane(
+                (mfh_u32)((double)(mfh_u32)c * (group.inverse * (double)CHUNK)));
+            if (step != Int4Group::kWide) {
+                const int r = (int)((mfh_u32)e0 - q * step);
+                const int on = r >= (int)step ? 1 : r < 0 ? -1 : 0;
+                g0 = (mfh_i64)q + on;
+                x0 = (mfh_u32)(r - on * (int)step);
+            } else {
+                mfh_i64 r = e0 - (mfh_i64)q * group.size;
+                const int on = r >= group.size ? 1 : r < 0 ? -1 : 0;
+                g0 = (mfh_i64)q + on;
+                const mfh_i64 to_next = group.size - (r - on * group.size);
+                x0 = to_next >= (mfh_i64)Int4Group::kWide ? 0u : Int4Group::kWide - (mfh_u32)to_next;
+            }
         }
     }
 
@@ -287,7 +298,7 @@ MFH_DEV void dequant_int4(const mfh_u8* __restrict__ packed, const void* __restr
         const int last = (int)min<mfh_i64>(kChunk, nitems - first) - 1;
         constexpr mfh_u32 kItemBytes = kElems / 2, kScaleBytes = SDT == kFloat32 ? 4 : 2;
         const char* items = reinterpret_cast<const char*>(packed) + first * kItemBytes;
-        const Int4Scales<kElems, ANY> map(group, first * kElems);
+        const Int4Scales<kElems, kChunk * kElems, ANY> map(group, c);
         const char* group0 = static_cast<const char*>(scales) + map.g0 * kScaleBytes;
         mfh_u32 w[U], sb[U], sb1[U];
         int own[U];
@@ -1120,7 +1131,9 @@ struct Int4Launch {
         // (step 1, an element-loop group, has no 32-bit multiplier and needs none)
         const uint64_t range = uint64_t(1) << 32;
         group.mul = (mfh_u32)(range / group.step + (range % group.step != 0));
-        const bool small = size < elems;
+        // Smaller than an item, or (past 2^34 elements) more groups than the
+        // kernel numbers in 32 bits: element by element.
+        const bool small = size < elems || (group.shift < 0 && n / size >= (int64_t(1) << 32));
         const bool any = !small && group.shift < 0;
         const int64_t items = small ? n : std::max<int64_t>(n / elems, 1);
         const mfh_u8* p = static_cast<const mfh_u8*>(packed);

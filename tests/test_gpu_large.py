@@ -74,6 +74,28 @@ def test_int4_past_2_32(torch):
         assert torch.equal(out[lo:hi].view(torch.int16), want.view(torch.int16)), f"int4 mismatch in [{lo}, {hi})"
 
 
+@pytest.mark.parametrize("group", [100, 100001])
+def test_int4_any_group_past_2_32(torch, group):
+    # groups that are not a power of two: the group of an element past 2^32 and
+    # items that run over a group's end there
+    n = (1 << 32) + 3 * 100001 + 5
+    nbytes, ngroups = (n + 1) // 2, -(-n // group)
+    log(f"int4 -> bf16, n = {n} nibbles, group {group}")
+    g = torch.Generator(device="cuda").manual_seed(group)
+    packed = torch.randint(0, 256, (nbytes,), dtype=torch.uint8, device="cuda", generator=g)
+    scales = (torch.rand(ngroups, device="cuda", generator=g) * 0.015 + 0.005).to(torch.float16)
+    out = torch.empty(n, dtype=torch.bfloat16, device="cuda")
+    M.dequant_int4(out.data_ptr(), M.BFLOAT16, packed.data_ptr(), n, scales.data_ptr(), M.FLOAT16, group,
+                   stream())
+    for lo, hi in chunks(n):
+        b = packed[lo // 2:(hi + 1) // 2].to(torch.int16)
+        nib = torch.stack([b & 15, b >> 4], dim=1).reshape(-1)[:hi - lo]
+        q = (nib - 16 * (nib >= 8).to(torch.int16)).float()
+        s = scales[torch.arange(lo, hi, device="cuda") // group].float()
+        want = (q * s).to(torch.bfloat16)
+        assert torch.equal(out[lo:hi].view(torch.int16), want.view(torch.int16)), f"int4 mismatch in [{lo}, {hi})"
+
+
 def test_axpy_past_2_31(torch):
     n = (1 << 31) + 3
     log(f"axpy f32, n = {n}")
@@ -123,8 +145,8 @@ def test_int4_encode_round_trip_past_2_31(torch):
 
 @pytest.mark.parametrize("in_dt", [M.BFLOAT16, M.FLOAT64, M.INT8])
 def test_casts_to_f32_past_2_31(torch, in_dt):
-    # bf16 -> f32 (k_convert16_vec), f64 -> f32 (k_narrow_f64_vec) and
-    # int8 -> f32 (k_convert_vec, two items per thread) over an odd count past
+    # bf16 -> f32 (k_convert_vec), f64 -> f32 (k_narrow_vec) and int8 -> f32
+    # (k_convert_vec, two items per thread) over an odd count past
     # 2^31: each is exact or one IEEE rounding (f64 -> f32 of finite values is
     # round-to-nearest-even, which torch's cast also does)
     n = (1 << 31) + 5
