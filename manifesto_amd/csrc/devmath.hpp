@@ -62,6 +62,9 @@
 #define mfh_absf(x) std::fabs((float)(x))
 #define mfh_maxf(a, b) std::fmax((float)(a), (float)(b))
 #define mfh_minf(a, b) std::fmin((float)(a), (float)(b))
+// NaN where an operand is one (IEEE 754-2019 minimum and maximum)
+inline float mfh_maximumf(float a, float b) { return std::isnan(a) || std::isnan(b) ? a + b : std::fmax(a, b); }
+inline float mfh_minimumf(float a, float b) { return std::isnan(a) || std::isnan(b) ? a + b : std::fmin(a, b); }
 #define mfh_is_nan_or_inf_class(v) (std::isnan(v) || std::isinf(v))
 inline unsigned mfh_fbits(float f) { unsigned u; __builtin_memcpy(&u, &f, 4); return u; }
 inline float mfh_fromfbits(unsigned u) { float f; __builtin_memcpy(&f, &u, 4); return f; }
@@ -98,6 +101,9 @@ extern "C" __device__ double __ocml_log_f64(double);
 #define mfh_absf(x) __builtin_fabsf(x)
 #define mfh_maxf(a, b) __builtin_fmaxf((a), (b))
 #define mfh_minf(a, b) __builtin_fminf((a), (b))
+// NaN where an operand is one (v_maximum3_f32, v_minimum3_f32)
+#define mfh_maximumf(a, b) __builtin_elementwise_maximum((a), (b))
+#define mfh_minimumf(a, b) __builtin_elementwise_minimum((a), (b))
 __device__ inline unsigned mfh_fbits(float f) { return __builtin_bit_cast(unsigned, f); }
 __device__ inline float mfh_fromfbits(unsigned u) { return __builtin_bit_cast(float, u); }
 __device__ inline int mfh_low_int(double d) { return (int)(unsigned)__builtin_bit_cast(unsigned long long, d); }
@@ -386,10 +392,9 @@ MFH_MATH float mfh_gelu_cr(float v, bool& rare)
 // value that the rounding test decides almost every element, in place of
 // library calls (codegen/cpu.go:177-185 evaluates math.Exp, math.Log and
 // math.Tanh in f64 and rounds once).  On MI355X, 2^24 elements: cap *
-// tanh(x / cap) over f32 27.5 us (78 with the library's f64 tanh), over bf16
-// 23 (77); log(e^x + 1) over f32 31 (60), over bf16 27 (56).  Still bound by
-// the f64 arithmetic (about 45 instructions per element for tanh), not by
-// the 19.5 and 9.7 us of the memory traffic.
+// tanh(x / cap) over f32 25.9 us (80 with the library's f64 tanh), over bf16
+// 22 (78); log(e^x + 1) over f32 33 (60), over bf16 30 (56).  Still bound by
+// the f64 arithmetic, not by the 19.7 and 9.9 us of the memory traffic.
 
 MFH_MATH float mfh_exp_ref(float v) { return (float)mfh_exp_f64((double)v); }
 MFH_MATH float mfh_log_ref(float v) { return (float)mfh_log_f64((double)v); }
@@ -405,26 +410,28 @@ MFH_MATH double mfh_exp_z(float m)
 }
 
 // The clamp changes no result: e^v rounds to 0 below -104 (e^-104 < 2^-150)
-// and to Inf above 89, which masked elements rely on.  Flagged: NaN and the
-// subnormal results in between, besides the undecided ones.
+// and to Inf above 89, which masked elements rely on, and NaN passes through
+// it.  Below 2^-126 (m < -87.3365) f32 keeps multiples of 2^-149: z + 2^-126
+// has the bits below those in its low 29, as z has above.  So only undecided
+// elements are flagged: e^v over bf16, 2^24 scores near -100, 16.4 us on MI355X
+// (44 with those flagged, 18 by the library).
 MFH_MATH float mfh_exp_cr(float v, bool& rare)
 {
-    const float m = mfh_med3f(v, -104.0f, 89.0f);
+    const float m = mfh_minimumf(mfh_maximumf(v, -104.0f), 89.0f);
     const double z = mfh_exp_z(m);
-    const float r = (float)z;
-    rare |= mfh_is_nan(v) | ((m > -104.0f) & (r <= 0x1p-126f)) | mfh_near_f32_midpoint(z, 1u << 15);
-    return r;
+    rare |= mfh_near_f32_midpoint(m < -87.33654f ? z + 0x1p-126 : z, 1u << 15);
+    return (float)z;
 }
 
-// log v for a positive normal v = 2^e m, m in [sqrt(1/2), sqrt(2)):
-// e ln2 + log m, log m = 2 atanh(s), s = (m - 1) / (m + 1), |s| < 0.1716, as
+// log(2^scale v) for a positive normal v = 2^e m, m in [sqrt(1/2), sqrt(2)):
+// (e + scale) ln2 + log m, log m = 2 atanh(s), s = (m - 1) / (m + 1), |s| < 0.1716, as
 // 2s + s^3 P(s^2) with P of degree 4 (the fit of gen_exp_poly.py, 2^-44.8
 // relative; e != 0 leaves at least 0.34 of the sum, so the relative error
 // stays below 2^-43).  m - 1 and m + 1 are exact.
-MFH_MATH double mfh_log_z(float v)
+MFH_MATH double mfh_log_z(float v, int scale)
 {
     const unsigned u = mfh_fbits(v) - 0x3f3504f3u;  // bits of sqrt(1/2)
-    const double e = (double)((int)u >> 23);
+    const double e = (double)(((int)u >> 23) + scale);
     const double m = (double)mfh_fromfbits((u & 0x7fffffu) + 0x3f3504f3u);
     const double s = (m - 1.0) * mfh_recip_newton(m + 1.0);
     const double y = s * s;
@@ -441,7 +448,7 @@ MFH_MATH double mfh_log_z(float v)
 // least 2^-41 of the value.
 MFH_MATH float mfh_log_cr(float v, bool& rare)
 {
-    const double z = mfh_log_z(v);
+    const double z = mfh_log_z(v, 0);
     rare |= !((v >= 0x1p-126f) & (v <= 0x1.fffffep127f)) | mfh_near_f32_midpoint(z, 1u << 12);
     return (float)z;
 }
@@ -471,15 +478,15 @@ MFH_MATH double mfh_tanh_z(float a)
 }
 
 // tanh v = v (1 - v^2 / 3 + ...) rounds to v up to 2^-12 (v^2 / 3 < 2^-25)
-// and to +-1 from 9.02 on, so neither end is flagged; NaN is.  The margin of
-// 2^13 f64 ulps is at least 2^-40 of the value.
+// and to +-1 from 9.02 on, so neither end is flagged, and NaN passes through.
+// The margin of 2^13 f64 ulps is at least 2^-40 of the value.
 MFH_MATH float mfh_tanh_cr(float v, bool& rare)
 {
-    const float a = mfh_minf(mfh_absf(v), 20.0f);
+    const float a = mfh_minimumf(mfh_absf(v), 20.0f);
     const double z = mfh_tanh_z(a);
     const bool self = a <= 0x1p-12f;
     const float r = mfh_fromfbits(mfh_fbits((float)z) | (mfh_fbits(v) & 0x80000000u));
-    rare |= mfh_is_nan(v) | (!self & mfh_near_f32_midpoint(z, 1u << 13));
+    rare |= !self & mfh_near_f32_midpoint(z, 1u << 13);
     return self ? v : r;
 }
 
@@ -526,9 +533,23 @@ MFH_RARE_FORM(sigmoid)
 MFH_RARE_FORM(silu)
 MFH_RARE_FORM(gelu)
 MFH_RARE_FORM(exp)
-MFH_RARE_FORM(log)
 MFH_RARE_FORM(tanh)
 #undef MFH_RARE_FORM
+// log's has the arguments that the rounding-tested form leaves out decided
+// without the library, subnormals as 2^-32 of a normal number (the log of a
+// vanished probability is ordinary data): 2^24 zeros in bf16 22 us on MI355X, 70
+// through the two forms (41 by the library inline).
+MFH_RARE float mfh_log_rare(float v)
+{
+    if (!((v > 0.0f) & (v <= 0x1.fffffep127f)))
+        return v == 0.0f ? mfh_fromfbits(0xff800000u) : v < 0.0f ? mfh_fromfbits(0x7fc00000u) : v + v;
+    const bool tiny = v < 0x1p-126f;
+    const double z = mfh_log_z(tiny ? v * 0x1p32f : v, tiny ? -32 : 0);
+    float s = (float)z;
+    MFH_KEEP(s);
+    if (mfh_near_f32_midpoint(z, 1u << 12)) s = mfh_log_ref(v);
+    return s;
+}
 MFH_FAST_OR_REF(mfh_sigmoid, mfh_sigmoid_fast, mfh_sigmoid_rare)
 MFH_FAST_OR_REF(mfh_silu, mfh_silu_fast, mfh_silu_rare)
 MFH_FAST_OR_REF(mfh_gelu, mfh_gelu_fast, mfh_gelu_rare)

@@ -5,6 +5,8 @@
 // The rounding-tested forms (<name>_p: mfh_<name>_cr, or the reference form
 // where it flags the input) add
 //   ref_mismatch=<bit patterns that differ from mfh_<name>_ref> flagged=<fraction>
+//   flagged_edge=<fraction over the arguments named in `edge` (Exp: results
+//     below the normal range, and NaN; Tanh: NaN), which data hold in masses>
 //   max_rel_err_log2=<log2 of the largest |z - f(v)| / |f(v)|>
 // where z is the f64 value the form rounds (mfh_<name>_z) and f(v) the same
 // formula in long double, over the inputs inside the form's range whose
@@ -20,6 +22,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <thread>
+#include <utility>
 #include <vector>
 
 static int64_t ulp_key(float f)
@@ -38,6 +41,7 @@ struct Fn {
     float (*ref)(float) = nullptr;        // the reference form it must reproduce,
     double (*z)(float) = nullptr;         // the f64 value it rounds (NaN outside its range)
     long double (*exact)(long double) = nullptr;
+    std::vector<std::pair<uint32_t, uint32_t>> edge = {};  // bit patterns, inclusive
 };
 
 // The rounding-tested forms' f64 values, inside each form's argument range.
@@ -67,7 +71,7 @@ static long double gelu_exact(long double v)
 }
 
 static double exp_z(float v) { return v >= -104.0f && v <= 89.0f ? mfh_exp_z(v) : NAN; }
-static double log_z(float v) { return v >= 0x1p-126f && v <= 0x1.fffffep127f ? mfh_log_z(v) : NAN; }
+static double log_z(float v) { return v >= 0x1p-126f && v <= 0x1.fffffep127f ? mfh_log_z(v, 0) : NAN; }
 // past 2^-12; below it the form gives v itself
 static double tanh_z(float v)
 {
@@ -95,9 +99,12 @@ int main(int argc, char** argv)
         {"sigmoid_p", 15, mfh_sigmoid_p, 1, mfh_sigmoid_cr, mfh_sigmoid_ref, sigmoid_z, sigmoid_exact},
         {"silu_p", 17, mfh_silu_p, 1, mfh_silu_cr, mfh_silu_ref, silu_z, silu_exact},
         {"gelu_p", 18, mfh_gelu_p, 1, mfh_gelu_cr, mfh_gelu_ref, gelu_z, gelu_exact},
-        {"exp_p", 12, mfh_exp_p, 1, mfh_exp_cr, mfh_exp_ref, exp_z, exp_exact},
+        {"exp_p", 12, mfh_exp_p, 1, mfh_exp_cr, mfh_exp_ref, exp_z, exp_exact,
+         {{0xc2ae0000u, 0xc2d20000u}, {0x7f800001u, 0x7fffffffu}}},
+        {"log_rare", 13, mfh_log_rare, 1, mfh_log_cr, mfh_log_ref, log_z, log_exact},
         {"log_p", 13, mfh_log_p, 1, mfh_log_cr, mfh_log_ref, log_z, log_exact},
-        {"tanh_p", 16, mfh_tanh_p, 1, mfh_tanh_cr, mfh_tanh_ref, tanh_z, tanh_exact},
+        {"tanh_p", 16, mfh_tanh_p, 1, mfh_tanh_cr, mfh_tanh_ref, tanh_z, tanh_exact,
+         {{0x7f800001u, 0x7fffffffu}}},
     };
     const char* only = argc > 3 ? argv[3] : nullptr;
     for (const Fn& f : fns) {
@@ -156,11 +163,25 @@ int main(int argc, char** argv)
             fl += flagged[w];
             mr = max_rel[w] > mr ? max_rel[w] : mr;
         }
+        int64_t edge_n = 0, edge_flagged = 0;
+        for (const auto& e : f.edge)
+            for (uint64_t u = e.first; u <= e.second; u += 13) {
+                const uint32_t bits = (uint32_t)u;
+                float v;
+                std::memcpy(&v, &bits, 4);
+                bool rare = false;
+                (void)f.cr(v, rare);
+                edge_n++;
+                edge_flagged += rare;
+                const float got = f.fn(v), r = f.ref(v);
+                if (bits_of(got) != bits_of(r) && !(std::isnan(got) && std::isnan(r))) rb++;
+            }
         std::printf("%s max_ulp=%lld over_tol=%lld nan_mismatch=%lld exact=%.6f samples=%lld", f.name,
                     (long long)m, (long long)o, (long long)nb, (double)ex / (double)n, (long long)n);
         if (f.cr)
             std::printf(" ref_mismatch=%lld flagged=%.6f max_rel_err_log2=%.2f", (long long)rb, (double)fl / (double)n,
                         mr > 0.0 ? std::log2(mr) : -1100.0);
+        if (edge_n) std::printf(" flagged_edge=%.6f", (double)edge_flagged / (double)edge_n);
         std::printf("\n");
     }
     return 0;
