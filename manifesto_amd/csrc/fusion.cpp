@@ -702,12 +702,14 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     // Vector loop: loads of all items first, then compute and store, at any
     // element alignment of the buffers (mfh_u32x4_any).
     //
-    // A periodic row of P elements is read at the item's index in it.  Where P
-    // is not a power of two the index takes mfh_row_index (a scalar remainder
-    // per wave and a 32-bit one per lane).  Where P is not a multiple of the
-    // item either, an item that runs over the row's end loads the row's last
+    // A periodic row of P elements is read at the item's index in it, a 64-bit
+    // remainder by a constant.  Where P is not a multiple of the item, that
+    // index takes mfh_row_index (a scalar remainder per wave and a 32-bit one
+    // per lane), an item that runs over the row's end loads the row's last
     // whole item instead and is filled element by element afterwards, a
-    // branch that one item in P / vec takes.  The element loop, one 2-byte
+    // branch that one item in P / vec takes.  (On rows of whole items the
+    // scalar remainder only held up the row's load: gelu(x + row) + r over f16
+    // [2048, 14336] 29.4 us with it, 28.6 without.)  The element loop, one 2-byte
     // access per lane, took 77 us for bias + gelu + residual over bf16
     // [8190, 2730] on MI355X, this loop 24; silu(gate) * up over bf16 buffers
     // one element off 16 bytes 58 us against 19.5 (16.5 aligned: a wave's
@@ -732,7 +734,7 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
         const std::string to = packed16[k] ? "w" + ks + "[u]" : "a" + ks + "[u]";
         const int64_t period = inputs[k].period;
         std::string index = operand_index(inputs[k], "e0");
-        if (inputs[k].mode == MFH_OPERAND_PERIODIC && !power_of_two(period))
+        if (row_ends(k) && !power_of_two(period))
             index = "mfh_row_index<" + std::to_string(period) + "ull>(e0)";
         if (row_ends(k)) {
             const std::string row = "row" + ks + "[u]";
