@@ -618,10 +618,16 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     // MFH_FUSION_PRECISE): two items per thread give a tanh chain 4%, an exp
     // and log chain 4% over f32 and 1% over bf16, a sigmoid chain 0-3% and the
     // precise SwiGLU chain 5.6% (the precise gelu chain -1%, within the noise
-    // of six alternating runs).  f32 chains of two or more full operands have
-    // 32 bytes per lane in flight with one item and take one: silu(gate) * up
-    // over f32 [2048, 14336] 54.6 us against 56.7 with two, [512, 32000] 31.7
-    // against 33.2.  SwiGLU, Silu, add/mul chains and (since its 2^f runs on
+    // of six alternating runs).  Where items are four elements and two or more
+    // operands are full, one item already has enough bytes in flight if it
+    // reads 32 (two f32 operands) or writes f32, and two cost occupancy.
+    // silu(a) * b on MI355X, 2^24 elements, one and two items: f32 * f32 -> f32
+    // 32.5 and 34.7 us, f32 * f32 -> bf16 28.0 and 29.6, bf16 * bf16 -> f32 26.7
+    // and 27.8, but f32 * bf16 -> bf16 26.1 and 24.6 and bf16 * bf16 + an f32 row
+    // -> bf16 25.3 and 23.6.  Sigmoid, Exp, Tanh and Gelu go the same way
+    // except gelu(a) * b over f32 * bf16 -> f32 (30.1 and 29.5: two), and Log
+    // gains nothing from two in any of these (f32 * bf16 -> bf16 25.4 and 29.5).
+    // SwiGLU, Silu, add/mul chains and (since its 2^f runs on
     // v_exp_f32) the gelu chain over 16 bits lose 2-6% with two, and the
     // reference forms inline (MFH_FUSION_NO_ROUNDING_TEST) gain nothing.
     // Workgroups of one wave (kFusedThreads).  mfh_set_launch_config("fused",
@@ -635,22 +641,25 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     // MFH_FUSION_NO_ROUNDING_TEST asks for the reference forms inline.
     const bool streams_f32 = vec == 4 && (flags & MFH_FUSION_SHORT_QUOTIENT) == 0;
     const bool rounded = precise ? (flags & MFH_FUSION_NO_ROUNDING_TEST) == 0 : streams_f32;
-    bool f64_fast = false;
-    for (const mfh_ast_node& node : list)
+    bool f64_fast = false, has_gelu = false, has_log = false;
+    for (const mfh_ast_node& node : list) {
         if (is_fast_activation(node.type) ? rounded || (!precise && node.type == kNodeSigmoid)
                                           : is_transcendental(node.type) && (rounded || !precise))
             f64_fast = true;
-    int full_operands = 0;
-    for (int k = 0; k < n_inputs; k++) full_operands += inputs[k].mode == MFH_OPERAND_FULL;
-    const bool two_items = f64_fast && !(vec == 4 && full_operands >= 2);
-    const int unroll = items_per_thread(Kern::kFused) > 0 ? items_per_thread(Kern::kFused) : two_items ? 2 : 1;
+        has_gelu |= node.type == kNodeGelu;
+        has_log |= node.type == kNodeLog;
+    }
+    int full_operands = 0, read_bytes = 0;  // bytes per element of the full operands
+    for (int k = 0; k < n_inputs; k++)
+        if (inputs[k].mode == MFH_OPERAND_FULL) full_operands++, read_bytes += inputs[k].dtype == kFloat32 ? 4 : 2;
+    const bool mixed = read_bytes != 2 * full_operands;  // (all f32 reads 32 bytes per item)
+    const bool one_item = !f64_fast || (vec == 4 && full_operands >= 2 &&
+                                        (read_bytes >= 8 || has_log || (out_dtype == kFloat32 && !(mixed && has_gelu))));
+    const int unroll = items_per_thread(Kern::kFused) > 0 ? items_per_thread(Kern::kFused) : one_item ? 1 : 2;
     const int auto_bpc = kOneShotBlocksPerCu;
     const int block = threads_per_block(Kern::kFused) > 0 ? threads_per_block(Kern::kFused) : kFusedThreads;
     // Non-temporal loads for the streamed (full-length) operands when the
     // kernel reads at least as many bytes per element as it writes.
-    int read_bytes = 0;
-    for (int k = 0; k < n_inputs; k++)
-        if (inputs[k].mode == MFH_OPERAND_FULL) read_bytes += inputs[k].dtype == kFloat32 ? 4 : 2;
     const bool stream_loads = read_bytes >= (out_dtype == kFloat32 ? 4 : 2);
 
     // Element loop: every operand decoded to f32.  Vector loop: f16 operands

@@ -148,7 +148,7 @@ def test_emit_hip_broadcast_operands():
     assert "mfh_gelu_fast(t1, qe)" in src and "mfh_gelu_rare(f1)" in src
     # gelu + residual can cancel: f16 output, so the guard's factor is 0.7 * 2^12 / 2
     assert src.count("qe |= !(mfh_absf(t3) * 1433.0f >= mfh_absf(t2));") == 2
-    # one item per thread; only a Sigmoid (mostly f64 work) takes two by default
+    # one item per thread; chains of mostly f64 work (a Sigmoid) take two by default
     assert "8 elements per item, 1 item(s) per thread" in src
     sig = M.FusedKernel(flatten((N_SIGMOID, ("in", 0))), [(M.FLOAT16, M.OPERAND_FULL, 0)], M.FLOAT16, "sig")
     assert "8 elements per item, 2 item(s) per thread" in sig.source
