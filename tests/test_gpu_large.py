@@ -125,6 +125,23 @@ def test_fused_chain_past_2_31(torch):
         assert torch.equal(out[lo:hi].view(torch.int16), want.view(torch.int16)), f"chain mismatch in [{lo}, {hi})"
 
 
+@pytest.mark.parametrize("period, n", [(2730, (1 << 32) + 4099), ((1 << 31) + 11, (1 << 31) + (1 << 16) + 5)])
+def test_periodic_row_past_2_31(torch, period, n):
+    # x + row: a short row indexed past 2^32 elements, and a row longer than
+    # 2^31, whose index takes 64 bits; both end inside items
+    log(f"fused Add(in0, row) bf16, n = {n}, period {period}")
+    k = M.FusedKernel(O.flatten((O.N_ADD, ("in", 0), ("in", 1))),
+                      [(M.BFLOAT16, M.OPERAND_FULL, 0), (M.BFLOAT16, M.OPERAND_PERIODIC, period)], M.BFLOAT16, "large_row")
+    g = torch.Generator(device="cuda").manual_seed(37)
+    x = torch.empty(n, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    row = torch.empty(period, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    out = torch.empty(n, dtype=torch.bfloat16, device="cuda")
+    k.launch([x.data_ptr(), row.data_ptr()], out.data_ptr(), n, stream())
+    for lo, hi in chunks(n):
+        want = (x[lo:hi].float() + row[torch.arange(lo, hi, device="cuda") % period].float()).to(torch.bfloat16)
+        assert torch.equal(out[lo:hi].view(torch.int16), want.view(torch.int16)), f"row mismatch in [{lo}, {hi})"
+
+
 def test_int4_encode_round_trip_past_2_31(torch):
     # int8 -> Int4 (int4Encode's clamp) -> int8 again over an odd count past
     # 2^31: the round trip must give every value clamped to [-8, 7] and the
