@@ -87,8 +87,8 @@ def wide_source(in_dt, n, rng):
 @pytest.mark.parametrize("in_dt", [O.FLOAT64, O.FLOAT32, O.INT64, O.INT32, O.UINT64, O.UINT32])
 @pytest.mark.parametrize("n, pad", [(50001, 0), (50001, 1), (50001, 8), (7, 0), (3, 2)])
 def test_wide_sources_tails_misaligned(in_dt, out_dt, n, pad):
-    # aligned buffers take whole items plus an element tail; a source or an
-    # output off its alignment runs the element loop
+    # whole items plus an element tail, with the source and the output on and
+    # off their alignment
     a = wide_source(in_dt, n, np.random.default_rng(in_dt * 11 + n + pad))
     got = convert(a, in_dt, out_dt, a.size, pad_in=pad, pad_out=pad % 3)
     check(got, ORACLE[out_dt](in_dt, a), f"{in_dt}->{out_dt} n={a.size} pad={pad}")
@@ -97,8 +97,8 @@ def test_wide_sources_tails_misaligned(in_dt, out_dt, n, pad):
 @pytest.mark.parametrize("out_pad", [0, 1, 2, 8, 16])
 @pytest.mark.parametrize("in_dt", [O.FLOAT16, O.INT16])
 def test_int8_from_2byte_sources_every_output_alignment(in_dt, out_pad):
-    # 2-byte sources write one 8-byte store per 16-byte source piece when the
-    # output is 8-byte aligned and run the 16-element items otherwise
+    # 2-byte sources write one 8-byte store per 16-byte source piece, at any
+    # output address
     n = 3 * 4096 + 37
     a = np.random.default_rng(out_pad).integers(0, 1 << 16, n, dtype=np.uint32).astype(np.uint16).view(NP_OF[in_dt])
     got = convert(a, in_dt, O.INT8, n, pad_out=out_pad)
@@ -185,9 +185,8 @@ def test_int4_from_every_code(in_dt):
 @pytest.mark.parametrize("in_dt", [O.FLOAT64, O.FLOAT32, O.INT64, O.INT32, O.UINT64, O.UINT32])
 @pytest.mark.parametrize("n, pad", [(50001, 0), (50001, 1), (50000, 16), (7, 0), (1, 2), (33, 0)])
 def test_int4_wide_sources_odd_counts_misaligned(in_dt, n, pad):
-    # 32-element items into 16-byte stores when the output is 16-byte
-    # aligned, the byte loop otherwise and for the tail; an odd count's last
-    # high nibble is 0
+    # whole source pieces at any address, then the bytes that are left; an odd
+    # count's last high nibble is 0
     a = wide_source(in_dt, n, np.random.default_rng(in_dt * 13 + n + pad))
     for m in (a.size, a.size - 1):  # both parities of the count
         got = convert_i4(a, in_dt, m, pad_in=pad, pad_out=pad % 3)

@@ -225,8 +225,8 @@ def test_convert_f32_narrowing_rounding_classes(out_dt):
 @pytest.mark.parametrize("out_dt", [O.FLOAT32, O.BFLOAT16, O.FLOAT16])
 @pytest.mark.parametrize("n, pad", [(50001, 0), (50001, 1), (7, 0), (3, 0)])
 def test_convert_other_numeric_dtypes(in_dt, np_dt, out_dt, n, pad):
-    # aligned sources take whole 16-byte output items plus an element tail;
-    # a source one byte off its alignment runs the element loop
+    # whole 16-byte output items (or source pieces) plus an element tail, from
+    # a source on its alignment or one byte off
     rng = np.random.default_rng(in_dt * 7 + n)
     raw = rng.integers(0, 256, size=8 * n, dtype=np.uint8)
     a = raw.view(np_dt)[:n]

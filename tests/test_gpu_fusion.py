@@ -35,14 +35,17 @@ def gpu():
     M.init(0)
 
 
-def run_fused(nodes, operands, arrays, out_dt, count, flags=0, pads=None, name="f"):
+def run_fused(nodes, operands, arrays, out_dt, count, flags=0, pads=None, name="f", off=0):
     """Compiles and launches one fusion; arrays are storage arrays.  `pads`
     offsets each buffer by whole elements (so 16-byte alignment is lost but
-    element alignment is kept); the output gets the first input's offset."""
+    element alignment is kept: whole items all the same) and `off` the full and
+    periodic ones and the output by bytes (the element loop, where that is off
+    an element); the output gets the first input's offset."""
     k = M.FusedKernel(nodes, operands, out_dt, name, flags)
     pads = pads or [0] * len(arrays)
-    devs = [to_dev(a, pad=p * a.itemsize) for a, p in zip(arrays, pads)]
-    out_pad = (pads[0] if pads else 0) * SIZE[out_dt]
+    devs = [to_dev(a, pad=p * a.itemsize + (off if o[1] != M.OPERAND_SCALAR else 0))
+            for a, p, o in zip(arrays, pads, operands)]
+    out_pad = (pads[0] if pads else 0) * SIZE[out_dt] + off
     out, op = empty_dev(count * SIZE[out_dt], pad=out_pad)
     k.launch([p for _, p in devs], op, count, stream())
     got = to_host(out, NP[out_dt], pad=out_pad)
@@ -182,13 +185,14 @@ def test_constants_and_deep_tree():
 
 @pytest.mark.parametrize("in_dt, out_dt", [(O.BFLOAT16, O.BFLOAT16), (O.FLOAT16, O.FLOAT16),
                                            (O.BFLOAT16, O.FLOAT32), (O.FLOAT32, O.FLOAT16)])
-@pytest.mark.parametrize("count, pad", [(8 * 1000, 0), (8 * 1000 + 5, 0), (3, 0), (10001, 2)])
-def test_storage_dtypes_tails_misaligned(in_dt, out_dt, count, pad):
+@pytest.mark.parametrize("count, pad, off", [(8 * 1000, 0, 0), (8 * 1000 + 5, 0, 0), (3, 0, 0), (10001, 2, 0),
+                                             (10001, 0, 1)])
+def test_storage_dtypes_tails_misaligned(in_dt, out_dt, count, pad, off):
     nodes = O.flatten((O.N_ADD, (O.N_MUL, (O.N_SILU, ("in", 0)), ("in", 1)), ("const", -0.5)))
     rng = np.random.default_rng(count + pad)
     g = O.encode(rng.normal(0, 2, count).astype(np.float32), in_dt)
     u = O.encode(rng.normal(0, 2, count).astype(np.float32), in_dt)
-    got = run_fused(nodes, [(in_dt, 0, 0)] * 2, [g, u], out_dt, count, pads=[pad, pad])
+    got = run_fused(nodes, [(in_dt, 0, 0)] * 2, [g, u], out_dt, count, pads=[pad, pad], off=off)
     gf, uf = O.decode(g, in_dt), O.decode(u, in_dt)
     silu = O.eval_unary(O.N_SILU, gf)
     tail = lambda s: O.encode((s * uf).astype(np.float32) + np.float32(-0.5), out_dt)  # noqa: E731
@@ -279,15 +283,16 @@ def test_gelu_chain_config4_full_size(flags):
 @pytest.mark.parametrize("act", [O.N_GELU, O.N_SILU])
 @pytest.mark.parametrize("out_dt", [O.FLOAT16, O.BFLOAT16])
 @pytest.mark.parametrize("op", [O.N_ADD, O.N_SUB])
-@pytest.mark.parametrize("count, pad", [(8 * 8192, 0), (8 * 8192 + 5, 1)])
-def test_cancellation_after_a_fast_activation_within_one_storage_ulp(act, out_dt, op, count, pad):
+@pytest.mark.parametrize("count, pad, off", [(8 * 8192, 0, 0), (8 * 8192 + 5, 1, 0), (8 * 8192 + 5, 0, 1)])
+def test_cancellation_after_a_fast_activation_within_one_storage_ulp(act, out_dt, op, count, pad, off):
     # act(v) + r (or - r) where r is the activation's value rounded to the
     # storage dtype, give or take two storage ulps, on three elements in four:
     # the sum is the activation's own rounding error, so a 2-ulp f32 node
     # error would be many storage ulps of it (an f16 denormal, typically).
     # The cancellation guard sends those elements to the reference form, and
     # every result stays within one storage ulp of the oracle.  pad > 0 loses
-    # the 16-byte alignment, so the element loop's guard runs instead.
+    # the 16-byte alignment; off > 0 the elements' own, so the element loop's
+    # guard runs instead.
     rng = np.random.default_rng(7000 + 97 * act + 13 * out_dt + op + count + pad)
     v = O.encode(rng.normal(0, 2, count).astype(np.float32), out_dt)
     vf = O.decode(v, out_dt)
@@ -299,7 +304,7 @@ def test_cancellation_after_a_fast_activation_within_one_storage_ulp(act, out_dt
     r[free] = O.encode(rng.normal(0, 2, int(free.sum())).astype(np.float32), out_dt)
     nodes = O.flatten((op, (act, ("in", 0)), ("in", 1)))
     got = run_fused(nodes, [(out_dt, M.OPERAND_FULL, 0)] * 2, [v, r], out_dt, count, pads=[pad, pad],
-                    name="cancel")
+                    name="cancel", off=off)
     want = O.encode(O.run(nodes, [vf, O.decode(r, out_dt)], count), out_dt)
     worst = compare_storage(got, want, out_dt, 1, f"cancellation act {act} op {op} out {out_dt} n {count}")
     exact = float(np.mean(got.view(np.uint16) == want.view(np.uint16)))
@@ -308,7 +313,7 @@ def test_cancellation_after_a_fast_activation_within_one_storage_ulp(act, out_dt
 
 
 def test_periodic_operand_not_multiple_of_8():
-    # period 12 forces the element-wise path; results must still match.
+    # a row that is not a multiple of a 16-bit item, here of f32 items
     nodes = O.flatten((O.N_ADD, ("in", 0), ("in", 1)))
     rng = np.random.default_rng(4)
     x = rng.normal(size=12 * 1000).astype(np.float32)

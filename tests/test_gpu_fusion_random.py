@@ -4,8 +4,10 @@ evaluator (CPUKernel.Run, codegen/cpu.go:59-214).
 Each seed draws a random FusionAST over every node type, 1-3 inputs in
 f32/bf16/f16 storage as full, periodic (a repeating row) or scalar operands,
 an element count that exercises the vector loop, its scalar tail or the
-element loop alone, and buffers that may be misaligned by one element.  Three
-classes of chain, each with a property that holds for every element:
+tail alone, and buffers that may be misaligned by one element.  Each case runs
+again on buffers one byte off, where the element loop takes the whole range,
+and must give the same bits.  Three classes of chain, each with a property that
+holds for every element:
 
 1. Default flags (the fast Sigmoid/Silu/Gelu forms and the cancellation
    guard), 16-bit outputs, chains in which every Sigmoid/Silu/Gelu reaches
@@ -24,7 +26,8 @@ classes of chain, each with a property that holds for every element:
    activations take their rounding-tested forms, the reference's values, so
    the same property as class 2 holds.
 
-Exp/Log/Tanh run the reference's f64 form in every mode.  Gelu's input goes
+Exp/Log/Tanh give the reference's f64 value, rounded once, in every mode
+(rounding-tested forms, the reference's where those cannot decide).  Gelu's input goes
 through Max(., -4.5): below -4.9 the reference's 1 + tanh(inner) cancels in
 f64 and its result is a multiple of 2^-53 |v|/2, which two correct f64
 evaluations may place one multiple apart (the single-node tests cover that
@@ -128,15 +131,23 @@ def run_case(tree, operands, arrays, values, periods, count, pad, out_dt, flags,
     log(f"seed {seed} flags {flags}: {describe(tree)} over {[(o[0], o[1], o[2]) for o in operands]}, "
         f"count {count} pad {pad} -> {out_dt}")
     k = M.FusedKernel(nodes, operands, out_dt, f"r{seed}", flags)
+    runs = []
     try:
-        # only full operands take the padding: periodic and scalar ones are read by index
-        devs = [to_dev(a, pad=(pad if o[1] == M.OPERAND_FULL else 0) * a.itemsize) for a, o in zip(arrays, operands)]
-        out_pad = pad * SIZE[out_dt]
-        out, op = empty_dev(count * SIZE[out_dt], pad=out_pad)
-        k.launch([p for _, p in devs], op, count, stream())
-        got = to_host(out, NP[out_dt], pad=out_pad)
+        for off in (0, 1):  # bytes
+            # only full operands take the padding: periodic and scalar ones are read by index
+            devs = [to_dev(a, pad=pad * a.itemsize + off if o[1] == M.OPERAND_FULL else 0)
+                    for a, o in zip(arrays, operands)]
+            out_pad = pad * SIZE[out_dt] + off
+            out, op = empty_dev(count * SIZE[out_dt], pad=out_pad)
+            k.launch([p for _, p in devs], op, count, stream())
+            runs.append(to_host(out, NP[out_dt], pad=out_pad))
     finally:
         k.close()
+    got, loop = runs
+    bits = np.uint32 if out_dt == O.FLOAT32 else np.uint16
+    gb, lb = got.view(bits), loop.view(bits)
+    differ = np.flatnonzero((gb != lb) & ~(nan_mask(gb, out_dt) & nan_mask(lb, out_dt)))
+    assert differ.size == 0, f"seed {seed}: the element loop differs at {differ[:3]}: {lb[differ[:3]]} from {gb[differ[:3]]}"
     want = O.encode(O.run(nodes, values, count, periods), out_dt)
     return got, want
 

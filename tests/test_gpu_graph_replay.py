@@ -307,40 +307,51 @@ def test_outputs_bound_over_inputs():
     same(tx, x + y, "s over x")
 
 
-def fresh_views(torch, n, pad):
-    """A new buffer of n floats, misaligned by one element when `pad`."""
-    store = torch.empty(n + 1, device="cuda")
-    return store[1:] if pad else store[:n]
+class FreshBuffer:
+    """A new buffer of n floats, `off` bytes off its allocation."""
+
+    def __init__(self, torch, n, off):
+        self.off, self.store = off, torch.empty(4 * n + 8, dtype=torch.uint8, device="cuda")
+        self.bytes = self.store[off:off + 4 * n]
+        self.value = (self.bytes.data_ptr(), M.FLOAT32, n)
+
+    def write(self, torch, a):
+        self.bytes.copy_(torch.from_numpy(a.view(np.uint8)))
+
+    def read(self):
+        return self.bytes.cpu().numpy().view(np.float32)
 
 
 @pytest.mark.parametrize("fuse", [False, True])
 def test_replays_on_fresh_buffers(fuse):
-    # New buffers on every call, every third one misaligned by one element, so
-    # that launches switch between the vector and the element path: calls 2
-    # onwards replay the captured graph with the changed launches rebound.
+    # New buffers on every call.  Every third one stands off its elements, so
+    # that launches switch between the vector loop and the element loop with
+    # its other grid; one output stands one element off on the calls between.
+    # Calls 2 onwards replay the captured graph with the changed launches
+    # rebound.
     torch = torch_mod()
     rng = np.random.default_rng(29 + fuse)
     g = chain_graph(fuse=fuse)
     n = (1 << 16) + 3
     for call in range(9):
-        pad = call % 3 == 2
+        off = 2 if call % 3 == 2 else 0
         x = rng.normal(0, 1, n).astype(np.float32)
         y = rng.normal(0, 1, n).astype(np.float32)
-        tx, ty = fresh_views(torch, n, pad), fresh_views(torch, n, pad)
-        te, tc = fresh_views(torch, n, pad), fresh_views(torch, n, not pad)
-        tx.copy_(torch.from_numpy(x))
-        ty.copy_(torch.from_numpy(y))
-        te.fill_(float("nan"))
-        tc.fill_(float("nan"))
+        bx, by, be = (FreshBuffer(torch, n, off) for _ in range(3))
+        bc = FreshBuffer(torch, n, 0 if off else 4)
+        bx.write(torch, x)
+        by.write(torch, y)
+        for b in (be, bc):
+            b.write(torch, np.full(n, np.nan, np.float32))
         torch.cuda.synchronize()
-        g.call({"x": tx, "y": ty}, {"e": te, "c": tc}, torch.cuda.current_stream().cuda_stream)
+        g.call({"x": bx.value, "y": by.value}, {"e": be.value, "c": bc.value}, torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
         want = chain_expected(x, y)
-        for k, t in (("e", te), ("c", tc)):
-            got = t.cpu().numpy()
+        for k, b in (("e", be), ("c", bc)):
+            got = b.read()
             bad = np.flatnonzero(got.view(np.uint32) != want[k].view(np.uint32))
-            assert bad.size == 0, f"call {call} (pad {pad}) output {k}: {bad.size} mismatches"
-        log(f"fresh-buffer call {call} (fused {fuse}, pad {pad}) ok")
+            assert bad.size == 0, f"call {call} (off {off}) output {k}: {bad.size} mismatches"
+        log(f"fresh-buffer call {call} (fused {fuse}, off {off}) ok")
     assert g.replayed_calls() == 7
 
 

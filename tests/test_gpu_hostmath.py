@@ -120,9 +120,7 @@ FLOATS = [O.FLOAT32, O.BFLOAT16, O.FLOAT16]
 @pytest.mark.parametrize("n, pad_in, pad_out", [(10007, 0, 0), (8, 0, 0), (3, 0, 0), (4099, 2, 0), (4099, 0, 4),
                                                 (4104, 8, 0)])
 def test_scalar_broadcast_vs_oracle(op, in_dt, out_dt, n, pad_in, pad_out):
-    # 16-byte output items where the buffers allow (an f32 source aligned to
-    # 16 bytes, a 16-bit one to the item's 8 or 16), the element loop
-    # otherwise and for the tail
+    # 16-byte output items at any address, the element loop for the tail
     rng = np.random.default_rng(5 + n + pad_in)
     src = O.encode(rng.normal(0, 10, n).astype(np.float32), in_dt)
     st, sp = to_dev(src, pad=pad_in)
