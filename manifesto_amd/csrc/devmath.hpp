@@ -398,7 +398,14 @@ MFH_MATH float mfh_gelu_cr(float v, bool& rare)
 
 MFH_MATH float mfh_exp_ref(float v) { return (float)mfh_exp_f64((double)v); }
 MFH_MATH float mfh_log_ref(float v) { return (float)mfh_log_f64((double)v); }
-MFH_MATH float mfh_tanh_ref(float v) { return (float)mfh_tanh_f64((double)v); }
+// The result is pinned: the compiler otherwise carries the library's copysign
+// through the conversions, and cannot select it from f16 to bf16 (it aborts).
+MFH_MATH float mfh_tanh_ref(float v)
+{
+    float r = (float)mfh_tanh_f64((double)v);
+    MFH_KEEP(r);
+    return r;
+}
 
 // e^m, m in [-104, 89]: 2^t, t = m log2(e), to 2^-39.8 (as mfh_sigmoid_z).
 MFH_MATH double mfh_exp_z(float m)
