@@ -96,8 +96,9 @@ int mfh_get_launch_config(const char* kernel, int32_t* blocks_per_cu, int32_t* i
 
 /* Threads per workgroup of a kernel family, the third part of its launch
  * shape.  "fp8", "axpy", "axpy16" and "convert" run 64, 128 or 256, "int4"
- * also 512 (defaults 128, 64, 64 and 512; "convert" picks per cast: 64 unless the
- * output is four times the source, then 256); "fused" takes any
+ * also 512 (defaults 128, 64, 64 and 512; "convert" picks per cast: 256 where the
+ * output is four times the source and for bytes from Int4, else 64; 16-bit
+ * "fp8" and "int4" outputs off their dwords run the defaults); "fused" takes any
  * power of two from 64 to 1024 and applies it to kernels compiled afterwards
  * (default 64, one wave).  The defaults are the fastest sizes measured on
  * MI355X.  0 keeps the current setting and -1 restores the default; also
