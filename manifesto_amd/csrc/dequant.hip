@@ -628,11 +628,12 @@ MFH_DEV mfh_u32 word_reg(const mfh_u32* w, int j)
 // workgroup.  Left to an element loop of the chunks' waves, what follows the
 // last chunk of a small cast was one serial chain: MI355X, 8190 elements
 // e4m3 -> e5m2 2.1 us (15.5 so), Int4 -> e4m3 1.9 (11.1), int8 -> Int4 1.95
-// (7.7), bf16 -> e4m3 2.0 (3.8).  Below kSpread pieces, about what fills the
-// chip's wave slots with one piece per lane, there are no chunks: 2^19
-// elements e4m3 -> e5m2 2.1 us (2.9 in chunks), bf16 -> e4m3 2.08 (2.16).
-// Large casts are unchanged but for Int4 ones that stay within the Infinity
-// Cache, 0.1-0.2 us longer (int8 -> Int4, 2^24 elements: 6.1, 5.9 before).
+// (7.7), bf16 -> e4m3 2.0 (3.8).  Below kSpread pieces, 2048 waves of one piece
+// per lane or two per SIMD, there are no chunks.  us in chunks and one piece
+// per lane, at 2^16, 2^17 and 2^18 pieces: e4m3 -> e5m2 3.13 and 2.27, 3.47 and
+// 2.99, 4.19 and 4.45; bf16 -> e4m3 2.16 and 2.06, 2.67 and 2.58, 3.10 and 3.43;
+// f32 -> e4m3 2.03 both, 2.02 and 2.15, 2.69 and 3.01; f64 -> int8 2.07 both,
+// 2.12 and 2.26, 2.28 and 2.75.
 struct WaveSplit {
     static constexpr int kChunk = 64 * 4;  // in pieces
     static constexpr mfh_i64 kSpread = 1 << 17;
