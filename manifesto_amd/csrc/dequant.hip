@@ -273,7 +273,7 @@ __global__ __launch_bounds__(BS) void k_dequant_int4_small(const mfh_u8* __restr
 // grid apart made the launch sweep U regions of the tensor at once, which on
 // this write-heavy mix ran 5.2 against 6.2 TB/s once the nibbles no longer
 // fit in the Infinity Cache.  bf16 from [4096, 14336] with an f32 scale per
-// row, MI355X: 22.1 us, against 110.8 by the element loop (2-byte
+// row, MI355X: 21.5 us, against 110.8 by the element loop (2-byte
 // stores, a 64-bit division per element), which every group that is not a
 // power of two took; with groups of 128 the shift runs 21.5 us where the
 // multiplication ran 21.6-21.9.
