@@ -89,7 +89,7 @@ int mfh_stream_sync(void* stream);
  * MFH_UNROLL_<KERNEL>.  "convert" reports 0 items per thread by default:
  * each cast picks its own (2 where the output is four times the source, else
  * 1; 4 runs as 2).  For "fused" the items per thread apply to kernels
- * compiled afterwards.  A deployment knob with no counterpart in the
+ * compiled afterwards, and launches too small to fill the chip use one.  A deployment knob with no counterpart in the
  * reference; results do not depend on it. */
 int mfh_set_launch_config(const char* kernel, int32_t blocks_per_cu, int32_t items_per_thread);
 int mfh_get_launch_config(const char* kernel, int32_t* blocks_per_cu, int32_t* items_per_thread);
