@@ -624,9 +624,11 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     // silu(a) * b on MI355X, 2^24 elements, one and two items: f32 * f32 -> f32
     // 32.5 and 34.7 us, f32 * f32 -> bf16 28.0 and 29.6, bf16 * bf16 -> f32 26.7
     // and 27.8, but f32 * bf16 -> bf16 26.1 and 24.6 and bf16 * bf16 + an f32 row
-    // -> bf16 25.3 and 23.6.  Sigmoid, Exp, Tanh and Gelu go the same way
-    // except gelu(a) * b over f32 * bf16 -> f32 (30.1 and 29.5: two), and Log
-    // gains nothing from two in any of these (f32 * bf16 -> bf16 25.4 and 29.5).
+    // -> bf16 25.3 and 23.6.  Sigmoid, Tanh and Gelu go the same way except
+    // gelu(a) * b over f32 * bf16 -> f32 (30.1 and 29.5: two).  Log gains nothing
+    // from two in any of these (f32 * bf16 -> bf16 25.4 and 29.5), nor does a chain
+    // of two full operands whose only f64 node is Exp, the lightest, at any width
+    // (e^a * b over bf16 18.8 and 19.0; 2^21 elements 4.5 and 4.8).
     // SwiGLU, Silu, add/mul chains and (since its 2^f runs on
     // v_exp_f32) the gelu chain over 16 bits lose 2-6% with two, and the
     // reference forms inline (MFH_FUSION_NO_ROUNDING_TEST) gain nothing.
@@ -641,11 +643,11 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     // MFH_FUSION_NO_ROUNDING_TEST asks for the reference forms inline.
     const bool streams_f32 = vec == 4 && (flags & MFH_FUSION_SHORT_QUOTIENT) == 0;
     const bool rounded = precise ? (flags & MFH_FUSION_NO_ROUNDING_TEST) == 0 : streams_f32;
-    bool f64_fast = false, has_gelu = false, has_log = false;
+    bool f64_fast = false, has_gelu = false, has_log = false, only_exp = true;
     for (const mfh_ast_node& node : list) {
         if (is_fast_activation(node.type) ? rounded || (!precise && node.type == kNodeSigmoid)
                                           : is_transcendental(node.type) && (rounded || !precise))
-            f64_fast = true;
+            f64_fast = true, only_exp &= node.type == kNodeExp;
         has_gelu |= node.type == kNodeGelu;
         has_log |= node.type == kNodeLog;
     }
@@ -653,8 +655,8 @@ int emit_hip(const mfh_ast_node* nodes, int n_nodes, const mfh_operand* inputs, 
     for (int k = 0; k < n_inputs; k++)
         if (inputs[k].mode == MFH_OPERAND_FULL) full_operands++, read_bytes += inputs[k].dtype == kFloat32 ? 4 : 2;
     const bool mixed = read_bytes != 2 * full_operands;  // (all f32 reads 32 bytes per item)
-    const bool one_item = !f64_fast || (vec == 4 && full_operands >= 2 &&
-                                        (read_bytes >= 8 || has_log || (out_dtype == kFloat32 && !(mixed && has_gelu))));
+    const bool enough_in_flight = vec == 4 && (read_bytes >= 8 || has_log || (out_dtype == kFloat32 && !(mixed && has_gelu)));
+    const bool one_item = !f64_fast || (full_operands >= 2 && (only_exp || enough_in_flight));
     const int unroll = items_per_thread(Kern::kFused) > 0 ? items_per_thread(Kern::kFused) : one_item ? 1 : 2;
     const int auto_bpc = kOneShotBlocksPerCu;
     const int block = threads_per_block(Kern::kFused) > 0 ? threads_per_block(Kern::kFused) : kFusedThreads;

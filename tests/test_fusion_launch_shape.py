@@ -25,7 +25,7 @@ def full(*dts):
     return [(dt, FULL, 0) for dt in dts]
 
 
-@pytest.mark.parametrize("node", [O.N_SIGMOID, O.N_SILU, O.N_EXP, O.N_TANH, O.N_GELU])
+@pytest.mark.parametrize("node", [O.N_SIGMOID, O.N_SILU, O.N_TANH, O.N_GELU])
 @pytest.mark.parametrize("operands, out, items", [
     (full(F, F), F, 1), (full(F, F), B, 1), (full(F, F, F), F, 1), (full(B, B), F, 1), (full(F, H), F, 1),
     # few bytes in flight per item
@@ -42,9 +42,11 @@ def test_items_per_thread_of_one_operand(node, dt, out):
     assert "4 elements per item, 2 item(s) per thread" in source((node, ("in", 0)), full(dt), out)
 
 
-@pytest.mark.parametrize("operands, out", [(full(F, B), B), (full(B, B) + [(F, ROW, 4096)], B)])
-def test_log_takes_one_item(operands, out):
-    assert "4 elements per item, 1 item(s) per thread" in product(O.N_LOG, operands, out)
+@pytest.mark.parametrize("node, operands, out", [
+    (O.N_LOG, full(F, B), B), (O.N_LOG, full(B, B) + [(F, ROW, 4096)], B),
+    (O.N_EXP, full(F, B), B), (O.N_EXP, full(F, F), F), (O.N_EXP, full(B, B), B)])
+def test_two_operands_of_a_log_or_an_exp_take_one_item(node, operands, out):
+    assert "elements per item, 1 item(s) per thread" in product(node, operands, out)
 
 
 # rows of whole items take the constant remainder; others the scalar one
